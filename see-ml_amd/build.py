@@ -33,6 +33,10 @@ DEVICE = [
     f"--offload-arch={ARCH}",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # The largest GEMM tile's epilogues pass the default size at which a
+    # requested full unroll is refused; rolled, they would index the
+    # accumulators at run time, from scratch memory.
+    "-mllvm", "-pragma-unroll-threshold=65536",
 ]
 
 

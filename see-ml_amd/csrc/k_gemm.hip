@@ -74,6 +74,55 @@ const char* GemmConfigName(int cfg) {
 // run. A forced skinny config still selects the outer kernel (tests).
 constexpr int64_t kSkinnyMaxRank = 16;
 
+namespace {
+// The tile of a GEMM by how many workgroups each leaves for the chip's 256
+// CUs. A larger tile reads its operands less often and splits them less per
+// product, and loses more to a last round of the chip that it leaves partly
+// idle. Measured on NT, one slice (us; 256x128 | 128x128 | 128x64 | 64x64):
+//   8192x2048x2048 339 | 358 | 430 | 452    2048x2048x2048 132 | 103 | 116 | 124
+//   2048x5504x2048 296 | 269 | 309 | 319    2048x1376x512   45 |  36 |  30 |  27
+//   2048x512x1376   87 |  63 |  44 |  31    600x4096x1024   75 |  60 |  53 |  45
+// So: 256x128 from rounds filled to 7/8 on, 128x128 from nearly a workgroup per
+// CU on, else 64x64 (the 128x64 tiles only where 64x64 would pass two per CU).
+int TileFor(const GemmDesc& d) {
+  if (d.N <= 32 && d.M > 32) return gemm::kCfgSkinnyN;
+  if (d.M <= 32 && d.N > 32) return gemm::kCfgSkinnyM;
+  auto tiles = [&](int64_t m, int64_t n) { return CeilDiv(d.M, m) * CeilDiv(d.N, n) * d.batch; };
+  constexpr int64_t kCus = 256, kMost = kCus * 7 / 8;
+  const int64_t large = tiles(256, 128);
+  if (d.causal == Causal::kNone && large * 8 >= CeilDiv(large, kCus) * kCus * 7) return gemm::kCfgLarge;
+  if (tiles(128, 128) >= kMost) return gemm::kCfgDefault;
+  if (tiles(128, 64) >= 2 * kMost) return gemm::kCfgHalf;
+  return gemm::kCfgSmall;
+}
+
+// Split-K slices, part of a shape's summation order. The rank-wide outputs of
+// the LoRA gradients (rowdot and colsum shapes, kind) have few tiles and a
+// long reduction, and so have outputs of at most 64 tiles: enough slices to
+// cover the chip twice with 64x64 or 128x128 tiles, each at least 128 deep.
+// Elsewhere a slice costs a pass over the output and a launch (about 5 us),
+// against about 0.6 us per 32 of depth that a lone workgroup takes: slices of
+// 1024 where the output leaves CUs idle (600x1024x1024 takes 24 us in one
+// slice, 600x1024x4096 82 us in one and 48 in four), otherwise none.
+int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
+  if (d.batch != 1 || d.causal != Causal::kNone || d.K < 256) return 1;
+  const int64_t big = CeilDiv(d.M, 128) * CeilDiv(d.N, 128), mid = CeilDiv(d.M, 64) * CeilDiv(d.N, 64);
+  int64_t tiles = mid;
+  if (kind == SkinnyKind::kRowDot || kind == SkinnyKind::kColSum || mid <= 64) {
+    tiles = d.N <= 32 && d.M > 32   ? CeilDiv(d.M, 128)
+            : d.M <= 32 && d.N > 32 ? CeilDiv(d.N, 128)
+            : big >= 512 || (mid < 256 && d.M > 64 && d.N > 64) ? big : mid;
+  } else if (mid < 256) {
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(d.K / 1024, 64)));
+  } else {
+    return 1;
+  }
+  if (tiles >= 512) return 1;
+  const int64_t want = CeilDiv(512, tiles), most = d.K / 128;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(most, 64))));
+}
+}  // namespace
+
 GemmPlan PlanGemmWith(const GemmDesc& d, int forced_cfg, int forced_splits) {
   GemmPlan plan;
   const SkinnyKind kind = SkinnyKindOf(d);
@@ -88,32 +137,12 @@ GemmPlan PlanGemmWith(const GemmDesc& d, int forced_cfg, int forced_splits) {
     plan.ws_bytes = SkinnyWorkspace(d);
     return plan;
   }
-  if (forced_cfg >= 0 && forced_cfg < kNumCfgs) {
-    plan.cfg = forced_cfg;
-  } else if (d.N <= 32 && d.M > 32) {
-    plan.cfg = gemm::kCfgSkinnyN;
-  } else if (d.M <= 32 && d.N > 32) {
-    plan.cfg = gemm::kCfgSkinnyM;
-  } else {
-    const int64_t big = CeilDiv(d.M, 128) * CeilDiv(d.N, 128) * d.batch;
-    const int64_t mid = CeilDiv(d.M, 64) * CeilDiv(d.N, 64) * d.batch;
-    plan.cfg = big >= 512 ? gemm::kCfgDefault
-               : (mid >= 256 || d.M <= 64 || d.N <= 64) ? gemm::kCfgSmall : gemm::kCfgDefault;
-  }
-  const CfgInfo& c = kCfgs[plan.cfg];
-  const int64_t tiles = CeilDiv(d.M, c.mt_m) * CeilDiv(d.N, c.mt_n) * d.batch;
-  int splits = 1;
-  const bool can_split = d.batch == 1 && d.causal == Causal::kNone;
-  if (forced_splits >= 1) {
-    splits = can_split ? forced_splits : 1;
-  } else if (can_split && tiles < 512 && d.K >= 256) {
-    // Enough workgroups to cover the chip twice, each slice >= 128 deep.
-    const int64_t want = CeilDiv(512, tiles);
-    const int64_t most = d.K / 128;
-    splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(most, 64))));
-  }
-  plan.splits = splits;
-  plan.ws_bytes = splits > 1 ? static_cast<size_t>(splits) * d.M * d.N * sizeof(float) : 0;
+  plan.cfg = forced_cfg >= 0 && forced_cfg < kNumCfgs ? forced_cfg : TileFor(d);
+  if (forced_splits >= 1)
+    plan.splits = d.batch == 1 && d.causal == Causal::kNone ? forced_splits : 1;
+  else
+    plan.splits = SplitsFor(d, kind);
+  plan.ws_bytes = plan.splits > 1 ? static_cast<size_t>(plan.splits) * d.M * d.N * sizeof(float) : 0;
   return plan;
 }
 
@@ -150,15 +179,12 @@ bool GemmPlanKeepsOrder(const GemmDesc& d, const GemmPlan& p) {
   return p.cfg >= 0 && p.cfg < kNumCfgs && p.splits == o.splits && (p.n_split == 0 || p.splits == 1);
 }
 
-// The heuristic plan, and for large GEMMs whose 256x128 tiles leave a
-// partial last round, the column split of at least two whole rounds with
-// the remainder on 64x64 tiles (the autotuner's first arm). The split was
-// 2-3% faster inside the C4 step on 8192x5504x2048 and 8192x32000x2048 with
-// a 128x128 remainder; 64x64 tiles spread the remainder over every CU
-// (8192x5504x2048: 1282 against 1319 us per pair, 128x64 1310).
+// The heuristic plan, and for large GEMMs whose 256x128 tiles leave much of a
+// last round idle, the column split of at least two whole rounds with the
+// remainder on 64x64 tiles (the autotuner's first arm).
 GemmPlan PlanGemm(const GemmDesc& d) {
   const GemmPlan plan = PlanGemmWith(d, -1, -1);
-  if (plan.cfg == kNumCfgs || plan.splits != 1) return plan;
+  if (plan.cfg == kNumCfgs || plan.cfg == gemm::kCfgLarge || plan.splits != 1) return plan;
   const GemmPlan sp = PlanGemmSplit(d, 2, gemm::kCfgSmall);
   const int64_t cus = DeviceCUs();
   if (sp.n_split > 0 && cus > 0 && CeilDiv(d.M, 256) * (sp.n_split / 128) >= 2 * cus) return sp;
@@ -166,7 +192,7 @@ GemmPlan PlanGemm(const GemmDesc& d) {
 }
 
 
-// Only the 256x128 tile, whose 108 KB of LDS holds one workgroup per CU, so
+// Only the 256x128 tile, of which one workgroup's registers fill a CU, so
 // a round of the chip is exactly one tile per CU.
 GemmPlan PlanGemmSplit(const GemmDesc& d, int cfg, int tail_cfg, int64_t n_split) {
   GemmPlan plan = PlanGemmWith(d, cfg, 1);
@@ -193,7 +219,7 @@ GemmPlan PlanGemmSplit(const GemmDesc& d, int cfg, int tail_cfg, int64_t n_split
 bool GemmVecForm(const GemmDesc& d) {
   return !d.b_int8 && VecOk(d.A, d.lda, d.a_sb, d.a_sh, d.a_kc ? d.K : d.M) &&
          VecOk(d.B, d.ldb, d.b_sb, d.b_sh, d.b_kc ? d.K : d.N) &&
-         d.lda < (int64_t{1} << 23) && d.ldb < (int64_t{1} << 23);
+         d.lda < (int64_t{1} << 22) && d.ldb < (int64_t{1} << 22);
 }
 
 // Validates a tile-kernel launch of d under plan (one column range, no
@@ -227,14 +253,14 @@ Status PrepareKArgs(const GemmDesc& d, const GemmPlan& plan, const Ctx& ctx, Gem
   // 16-byte vector loads need 16-byte alignment of every batch base and a
   // contiguous extent that is a multiple of 4 (a float4 is then wholly in or
   // out of range); per-lane offsets within a tile must fit 32 bits. Other
-  // GEMMs (int8 B, odd shapes) take the element-load form of the small tile.
+  // GEMMs (int8 B, odd shapes) take the general form of the plan's tile.
   const bool vec = GemmVecForm(d);
   if (d.out_scaled && (!d.out || !vec))
     return Status::Fail(kUnitEngine, "Gemm: a fused Scale + AddEW needs the 16-byte-load kernels");
   if (d.out && !vec && d.ldo && d.ldo != d.N)
     return Status::Fail(kUnitEngine, "Gemm: a column view's fused AddEW needs the 16-byte-load kernels");
   if (d.out && !vec) return Status::Fail(kUnitEngine, "Gemm: a fused AddEW needs the 16-byte-load kernels");
-  const int cfg = vec ? plan.cfg : gemm::kCfgSmall;
+  const int cfg = vec ? plan.cfg : gemm::GeneralCfg(plan.cfg);
   const CfgInfo& c = kCfgs[cfg];
   const int64_t tm = CeilDiv(d.M, c.mt_m), tn = CeilDiv(d.N, c.mt_n);
   // The kernel decomposes its linear workgroup id in 32 bits.

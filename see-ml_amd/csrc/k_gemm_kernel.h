@@ -16,22 +16,51 @@
 // zeroes.
 //
 // Mapping to CDNA4: a workgroup of 4 or 8 wavefronts (64 lanes) owns an
-// MT_M x MT_N output tile; each wavefront owns a WM x WN sub-tile accumulated
-// with v_mfma_f32_32x32x2_f32 (32x32 outputs, 16 accumulators per lane, two
-// k values per instruction, one per half-wavefront). Operand tiles
-// (KT = 32 or 64 per config) are staged through LDS, double-buffered:
-// the next stage's 16-byte global loads are in flight while the matrix cores
-// consume the current one. The k loop carries no per-element address math:
-// each lane's offsets from the stage origin are fixed at kernel entry (rows
-// past the operand's end are clamped onto its last row — their products
-// reach only outputs that are never stored), the origin advances by a
-// uniform step, and only a final partial stage masks k.
+// MT_M x MT_N output tile; each wavefront owns a WM x WN sub-tile of 32x32
+// blocks, 16 accumulators per lane each. Operand tiles (KT = 16 or 32 deep
+// per config) are staged through LDS, double-buffered: the next stages'
+// 16-byte global loads are in flight while the matrix cores consume the
+// current one. The k loop carries no per-element address math: each lane's
+// offsets from the stage origin are fixed at kernel entry (rows past the
+// operand's end are clamped onto its last row: their products reach only
+// outputs that are never stored), the origin advances by a uniform step, and
+// only a final partial stage masks k.
 //
-// k assignment: a fragment group covers 8 k. Half-wavefront h of MFMA j
-// (j = 0..3) supplies k = 8g + 4h + j, for A and B alike, so a k-contiguous
-// operand kept in LDS as [o][k] rows is read with ONE 16-byte ds_read per
-// lane per four MFMAs; an o-contiguous operand is kept as [k][o] rows and
-// read as four 4-byte reads (consecutive lanes, consecutive addresses).
+// Products. The fp32 MFMA (v_mfma_f32_32x32x2_f32) peaks at 157 TFLOP/s and
+// bounded every large GEMM here at 125-147; the bf16 MFMA runs 16x as many
+// products. An fp32 value is exactly the sum of three bf16 values (24
+// significand bits as 8 + 8 + 8, each part the round-to-nearest of what is
+// left: Split4), so a product is nine bf16 products, each exact in fp32. The
+// three smallest are at most 2^-26 of the whole, a quarter of the fp32
+// product's own rounding, and are left out; the other six run as six
+// v_mfma_f32_32x32x16_bf16 into one fp32 accumulator, smallest first. The
+// accumulator is added to a second one and cleared every 64 k (kChunk): the
+// bf16 MFMA's own additions lean slightly to one side, which a sum over many
+// rows of such results would show, and short sums keep that and the rounding
+// small. Relative 2-norm error against 64 bits, fp32 MFMA | this: normal
+// operands K = 16 7.4e-8 | 3.3e-8, K = 2048 8.1e-7 | 1.6e-7, K = 8192 1.62e-6 |
+// 2.5e-7; softmax gradients times a head of 8192 classes 1.6e-6 | 2.3e-7;
+// log-normal operands 6.6e-7 | 1.3e-7 (without the second accumulator 7.0e-7
+// on the second, and gradients summed over 2048 rows were further off than
+// with the fp32 MFMA). An int8 operand is one bf16 part: three products.
+// Measured: NT 8192x2048x5504 1330 -> 890 us, 8192x5504x2048 1340 -> 975 us,
+// 190-208 TFLOP/s of fp32 products where 157 was the fp32 MFMA's peak. What
+// bounds it now is power: the matrix cores are 76% busy at 1.74 GHz (2.4 with
+// little to do), and a loop of bf16 MFMAs alone on random bits runs at the
+// clock that makes 300.
+//
+// What the split cannot hold (an infinity or NaN, a value that rounds past
+// bf16's largest, a result so small that parts below 2^-133 matter) shows in
+// the accumulators: non-finite, or nonzero below 2^-100. A wavefront that
+// finds one in a 32x32 block computes that block again with the fp32 MFMA,
+// straight from memory (Recompute below), so non-finites propagate as fp32 products do.
+//
+// k assignment: half-wavefront h supplies k = 16g + 8h + 0..7 of the group
+// g of 16, for A and B alike. The split happens once per element and
+// workgroup, between the global load and the LDS store; LDS holds the three
+// parts as planes. A k-contiguous operand is kept as [o][k] rows and read
+// with one 16-byte ds_read per part, fragment and lane; a row-contiguous one
+// is kept as [k][o] rows and read with the transposing ds_read_b64_tr_b16.
 //
 // Workgroup order: the 8 XCDs (each with its own L2) receive workgroups
 // round-robin, so the linear workgroup id is remapped to give each XCD a
@@ -42,10 +71,10 @@
 // order is fixed by the tile loop; split-K writes per-slice partials that a
 // second kernel sums in slice order. No atomics.
 //
-// Numerics: fp32 products, fp32 accumulation in the matrix core (full
-// IEEE single precision, not a reduced-precision xf32 mode). The reference
-// accumulates in a different order (4-wide k groups / sequential), so GEMM
-// outputs agree to within fp32 reordering error, not bit-for-bit.
+// Numerics: operands held to all 24 bits, fp32 accumulation in the matrix
+// core (above). The reference accumulates in a different order (4-wide k
+// groups / sequential), so GEMM outputs agree to within fp32 reordering
+// error, not bit-for-bit.
 #pragma once
 
 #include "device_common.h"
@@ -58,20 +87,138 @@ namespace seeml_hip {
 namespace gemm {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint32u __attribute__((aligned(1)));
 
-constexpr int KG = 8;           // k covered by one fragment group
+constexpr int KG = 16;          // k covered by one MFMA
 constexpr int kXcds = 8;
 constexpr int kGroupRows = 8;   // tile-rows walked together (L2 panel sharing)
-constexpr int kSplitAlign = 64; // split-K slice depth: a multiple of every KT
+constexpr int kChunk = 64;      // k summed in the matrix core before a rounded fp32 addition
+constexpr int kSplitAlign = 64; // split-K slice depth: a multiple of kChunk and every KT
 
-// LDS row strides in floats. [o][k] rows of KT + 4: the 16-byte fragment
-// reads of 8 consecutive lanes (8 rows, same k) cover the 32 banks once.
-// [k][o] rows padded by 8: the half-wavefronts (k and k + 4) fall in
-// disjoint bank halves.
-constexpr int KcStride(int kt) { return kt + 4; }
-constexpr int RcStride(int mt) { return mt + 8; }
+// LDS layout of one part (plane) of an operand stage, in bf16 elements. A
+// 16-byte fragment read serves 16 lanes a cycle (64 banks). [o][k] rows of
+// KT with the 16-byte chunks of a row permuted by its row number, so that the
+// 16 rows read at one logical chunk fall in 16 different bank quads, without
+// padding. [k][o] rows padded to 64 bytes past a multiple of the banks: the
+// four rows of a transposing read's 32 lanes fall in disjoint quarters.
+// (Permuted by row pairs and padded by 32 bytes instead, every read took twice
+// its cycles: 36% of the LDS cycles at 8192x2048x5504 were conflicts.)
+template <int KT>
+__device__ __forceinline__ constexpr int KcChunk(int o, int c) {
+  return KT == 32 ? c ^ ((o >> 2) & 3) : c ^ ((o >> 3) & 1);
+}
+constexpr int RcStride(int mt) { return mt == 32 ? 32 : mt + 32; }
 template <int MT, int KT, bool KC>
-constexpr int TileFloats() { return KC ? MT * KcStride(KT) : KT * RcStride(MT); }
+constexpr int PlaneElems() { return KC ? MT * KT : KT * RcStride(MT); }
+
+// A wavefront-uniform pointer to global memory as one scalar value. Without
+// this the compiler reassociates (base + per-lane offset) + stage step and
+// keeps a 64-bit vector pointer per load in flight.
+template <typename T>
+using GlobalPtr = const __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ GlobalPtr<T> ScalarBase(const T* p) {
+  GlobalPtr<T> q = (GlobalPtr<T>)p;
+  asm("" : "+s"(q));
+  return q;
+}
+
+// x as three bf16 parts, x = part 0 + part 1 + part 2 exactly for every
+// finite x of at most bf16's range and at least 2^-110 (below, part 2 loses
+// what lies under 2^-133). Packed: part i of (x0, x1) in p[i].
+__device__ __forceinline__ void Split2(float x0, float x1, uint32_t (&p)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const bf16x2 h = __builtin_convertvector((floatx2){x0, x1}, bf16x2);
+    p[i] = __builtin_bit_cast(uint32_t, h);
+    if (i < 2) {
+      // What is left, exactly.
+      x0 -= __builtin_bit_cast(float, p[i] << 16);
+      x1 -= __builtin_bit_cast(float, p[i] & 0xFFFF0000u);
+    }
+  }
+}
+
+// The parts of a lane's 8 consecutive k.
+__device__ __forceinline__ void Split8(const float* x, bf16x8 (&f)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t p[3];
+    Split2(x[2 * q], x[2 * q + 1], p);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) w[part][q] = p[part];
+  }
+#pragma unroll
+  for (int part = 0; part < 3; ++part)
+    f[part] = __builtin_bit_cast(bf16x8, make_uint4(w[part][0], w[part][1], w[part][2], w[part][3]));
+}
+
+// One 16-deep step of a block of fragments into its accumulators: the six
+// products of NA = NB = 3 parts, or the three of an exact (one-part) B,
+// smallest first, each over all blocks so that consecutive MFMAs are
+// independent. FOLD: the first step of a chunk (kChunk): the accumulators,
+// holding the chunk before, are added to `sum` and start again from zero.
+template <bool FOLD, int BM, int BN, int PB>
+__device__ __forceinline__ void MfmaStep(const bf16x8 (&fa)[BM][3], const bf16x8 (&fb)[BN][PB],
+                                         floatx16 (&acc)[BM][BN], floatx16 (&sum)[BM][BN]) {
+  constexpr int kProducts = PB == 3 ? 6 : 3;
+  constexpr int ia[6] = {2, PB == 3 ? 0 : 1, PB == 3 ? 1 : 0, 1, 0, 0};
+  constexpr int ib[6] = {0, PB == 3 ? 2 : 0, PB == 3 ? 1 : 0, 0, PB == 3 ? 1 : 0, 0};
+  constexpr floatx16 kZero = {};
+#pragma unroll
+  for (int q = 0; q < kProducts; ++q)
+#pragma unroll
+    for (int i = 0; i < BM; ++i)
+#pragma unroll
+      for (int j = 0; j < BN; ++j) {
+        if (FOLD && q == 0) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) sum[i][j][v] += acc[i][j][v];
+        }
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            fa[i][ia[q]], fb[j][ib[q]], FOLD && q == 0 ? kZero : acc[i][j], 0, 0, 0);
+      }
+}
+
+// The issue order of one stage: kFirst fragment reads, then after each of the
+// kMfma MFMAs its share of the VALU operations that split kVecs vectors (22
+// each and their addresses), one LDS read, one LDS write and one global load.
+// Left to itself the scheduler issues the MFMAs first and the split after
+// them, so that a wavefront alone on its SIMD takes the sum of the two.
+template <int kMfma, int kVecs, int kFirst>
+__device__ __forceinline__ void Interleave() {
+  __builtin_amdgcn_sched_group_barrier(0x100, kFirst, 0);
+#pragma unroll
+  for (int q = 0; q < kMfma; ++q) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, (24 * kVecs + kMfma - 1) / kMfma, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+  }
+}
+
+// Whether any lane's accumulators hold what the split cannot vouch for: a
+// non-finite value, or a nonzero one below 2^-100. Uniform per wavefront.
+__device__ __forceinline__ bool AnySuspect(const floatx16& acc) {
+  uint32_t low = ~0u;  // min over (|c| bits << 1) - 1; zero wraps to the top
+  float nonfinite = 0.0f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const float c = acc[v];
+    low = std::min(low, (__builtin_bit_cast(uint32_t, c) << 1) - 1u);
+    nonfinite = __builtin_fmaf(c, 0.0f, nonfinite);
+  }
+  constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1u;
+  return __ballot(low < kTiny || !(nonfinite == 0.0f)) != 0;
+}
 
 struct GemmKArgs {
   const void* A;
@@ -141,26 +288,33 @@ struct CfgInfo {
   const char* name;
 };
 inline constexpr CfgInfo kCfgs[] = {
-    {128, 128, 32, 256, "128x128x32/w2x2"}, {128, 128, 32, 512, "128x128x32/w4x2"},
-    {256, 128, 32, 512, "256x128x32/w4x2"}, {128, 256, 32, 512, "128x256x32/w2x4"},
+    {128, 128, 16, 256, "128x128x16/w2x2"}, {128, 128, 16, 512, "128x128x16/w4x2"},
+    {256, 128, 16, 512, "256x128x16/w4x2"}, {128, 256, 16, 512, "128x256x16/w2x4"},
     {128, 64, 32, 256, "128x64x32/w2x2"},   {64, 64, 32, 256, "64x64x32/w2x2"},
     {128, 32, 32, 256, "128x32x32/w4x1"},   {32, 128, 32, 256, "32x128x32/w1x4"},
     {64, 128, 32, 256, "64x128x32/w2x2"},   {128, 64, 32, 256, "128x64x32/w4x1"},
-    {128, 128, 16, 256, "128x128x16/w2x2"}, {64, 128, 16, 256, "64x128x16/w2x2"},
+    {64, 64, 16, 256, "64x64x16/w2x2"},     {64, 128, 16, 256, "64x128x16/w2x2"},
 };
+// Wavefronts per SIMD to keep registers for: two of the large tiles'.
+constexpr int MinWaves(int mt_m, int mt_n) { return mt_m * mt_n >= 128 * 128 ? 2 : 1; }
 inline constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
-inline constexpr int kCfgDefault = 0, kCfgSmall = 5, kCfgSkinnyN = 6, kCfgSkinnyM = 7;
+inline constexpr int kCfgDefault = 0, kCfgSmall = 5, kCfgSkinnyN = 6, kCfgSkinnyM = 7,
+                     kCfgLarge = 2, kCfgHalf = 9;
 
 // One operand's MT x KT stage (outer index o = m for A / n for B), held in
-// registers between its global loads and its LDS store. KC = k-contiguous.
+// registers between its global loads and its LDS store, where it is split.
+// KC = k-contiguous. Vector i of a thread is 4 elements along the contiguous
+// direction.
 //
 // VEC (16-byte aligned rows, contiguous extent a multiple of 4): 16-byte
 // loads at per-lane offsets fixed for the whole k loop; the stage origin is
 // uniform. A final partial stage (k beyond the reduction's end) zeroes its
 // out-of-range vectors, reading the row start instead.
-// !VEC (int8 B, odd shapes): element loads with an in-range mask applied at
-// the LDS store. Both forms are branch-free per element, so a stage's loads
-// are all in flight together and the first wait is at the LDS store.
+// !VEC (any extent, stride and alignment; int8): the same vectors by loads
+// that need only the element's own alignment. Row-contiguous, a vector that
+// would pass the row's end is read back from the end and shifted into place
+// at the LDS store (an extent below 4: element loads); k-contiguous, a final
+// partial stage is read by elements. Out-of-range elements are zero.
 //
 // SC (VEC only): every loaded element in range is scaled, fl(sc * x), as a
 // Scale instruction would have stored it; zeros past the reduction's end
@@ -170,15 +324,26 @@ inline constexpr int kCfgDefault = 0, kCfgSmall = 5, kCfgSkinnyN = 6, kCfgSkinny
 // partial stage is scaled as loaded, under its in-range masks.
 template <int MT, int KT, bool KC, typename T, int NT, bool VEC, bool SC = false>
 struct Stage {
+  static constexpr bool kF32 = std::is_same<T, float>::value;
+  static constexpr int kParts = kF32 ? 3 : 1;
+  static constexpr int kPlane = PlaneElems<MT, KT, KC>();
+  static constexpr int kElems = kParts * kPlane;  // LDS elements of a stage
   static constexpr int kVecs = MT * KT / 4;
   static constexpr int kPer = kVecs / NT;
-  static_assert(kVecs % NT == 0 && kPer * 4 <= 64, "stage shape");
+  static_assert(kVecs % NT == 0, "stage shape");
   static_assert(!SC || VEC, "scaled loads need the vector form");
+  static_assert(!VEC || kF32, "int8 operands take the general form");
   float r[kPer][4];
-  uint32_t off[kPer];  // VEC: element offset of vector i from the stage origin
-  uint64_t ok;         // !VEC: bit 4i+e set when element e of vector i is in range
-  float sc;            // SC: the factor
-  bool pend;           // SC: loaded unscaled (a whole stage), scaled at the store
+  // Byte offset of vector i from the stage origin. VEC: the host checks that
+  // it fits 32 bits, so a load is a uniform base plus a 32-bit offset.
+  using Off = typename std::conditional<VEC, uint32_t, int64_t>::type;
+  static constexpr int kSize = sizeof(T);
+  Off off[kPer];
+  int shift[kPer];    // !VEC, row-contiguous: places the vector was read back by
+  int avail;          // !VEC, row-contiguous: elements of the row from the tile's start on
+  bool few;           // !VEC, row-contiguous: rows of fewer than 4 elements
+  float sc;           // SC: the factor
+  bool pend;          // SC: loaded unscaled (a whole stage), scaled at the store
 
   __device__ __forceinline__ static void coords(int v, int& o, int& k) {
     if constexpr (KC) {
@@ -192,106 +357,190 @@ struct Stage {
 
   // o0: first row of the tile (a multiple of 4); oe: the operand's extent.
   __device__ __forceinline__ void init(int64_t ld, int64_t o0, int64_t oe) {
-    if constexpr (VEC) {
-      const int64_t last = oe - o0 - (KC ? 1 : 4);  // >= 0: the tile starts in range
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        int o, k;
-        coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
-        const int64_t oc = std::min<int64_t>(o, last);
-        off[i] = static_cast<uint32_t>(KC ? oc * ld + k : k * ld + oc);
-      }
+    const int64_t left = oe - o0;  // >= 1: the tile starts in range
+    if constexpr (!VEC && !KC) {
+      avail = static_cast<int>(std::min<int64_t>(left, MT));
+      few = oe < 4;
     }
-  }
-
-  // A whole stage in range (VEC): one 16-byte load per vector, no masks.
-  __device__ __forceinline__ void load_full(const T* __restrict__ org) {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const float4 q = *reinterpret_cast<const float4*>(org + off[i]);
-      r[i][0] = q.x; r[i][1] = q.y; r[i][2] = q.z; r[i][3] = q.w;
-    }
-    if constexpr (SC) pend = true;
-  }
-
-  // Any stage: k beyond ke (and, for !VEC, rows beyond oe) read as zero.
-  __device__ __forceinline__ void load(const T* __restrict__ X, int64_t ld, int64_t o0,
-                                       int64_t oe, int64_t k0, int64_t ke) {
-    if constexpr (VEC) {
-      const T* org = X + (KC ? o0 * ld + k0 : k0 * ld + o0);
-      const int64_t kvalid = ke - k0;
-      if (kvalid >= KT) {
-        load_full(org);
-      } else {
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-          int o, k;
-          coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
-          const bool in = k < kvalid;  // a KC vector is wholly in or out (K % 4 == 0)
-          const int64_t back = KC ? k : static_cast<int64_t>(k) * ld;
-          float4 q = *reinterpret_cast<const float4*>(org + (off[i] - (in ? 0 : back)));
-          if constexpr (SC) q = make_float4(sc * q.x, sc * q.y, sc * q.z, sc * q.w);
-          if constexpr (SC) pend = false;
-          r[i][0] = in ? q.x : 0.0f;
-          r[i][1] = in ? q.y : 0.0f;
-          r[i][2] = in ? q.z : 0.0f;
-          r[i][3] = in ? q.w : 0.0f;
-        }
-      }
-    } else {
-      ok = 0;
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        int o, k;
-        coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
-        const int64_t go = o0 + o, gk = k0 + k;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t eo = KC ? go : go + e;
-          const int64_t ek = KC ? gk + e : gk;
-          const bool in = eo < oe && ek < ke;
-          r[i][e] = static_cast<float>(X[in ? (KC ? eo * ld + ek : ek * ld + eo) : 0]);
-          ok |= (in ? uint64_t{1} : uint64_t{0}) << (4 * i + e);
-        }
-      }
-    }
-  }
-
-  __device__ __forceinline__ void store(float* __restrict__ lds) const {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       int o, k;
       coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
-      float* dst = KC ? lds + o * KcStride(KT) + k : lds + k * RcStride(MT) + o;
-      float4 q;
-      if constexpr (VEC) {
-        q = make_float4(r[i][0], r[i][1], r[i][2], r[i][3]);
-        if constexpr (SC)
-          if (pend) q = make_float4(sc * q.x, sc * q.y, sc * q.z, sc * q.w);
+      int64_t oc = o;
+      if constexpr (KC) {
+        oc = std::min<int64_t>(o, left - 1);
+      } else if constexpr (VEC) {
+        oc = std::min<int64_t>(o, left - 4);
       } else {
-        q.x = (ok >> (4 * i + 0)) & 1 ? r[i][0] : 0.0f;
-        q.y = (ok >> (4 * i + 1)) & 1 ? r[i][1] : 0.0f;
-        q.z = (ok >> (4 * i + 2)) & 1 ? r[i][2] : 0.0f;
-        q.w = (ok >> (4 * i + 3)) & 1 ? r[i][3] : 0.0f;
+        // Back to the row's last 4 elements: at least 0 from the row's start.
+        oc = oe < 4 ? 0 : std::min<int64_t>(o, left - 4);
+        shift[i] = static_cast<int>(o - oc);
       }
-      *reinterpret_cast<float4*>(dst) = q;
+      off[i] = static_cast<Off>((KC ? oc * ld + k : k * ld + oc) * kSize);
+    }
+  }
+
+  // Vector i, `back` bytes before its place.
+  __device__ __forceinline__ void load_vec(int i, GlobalPtr<T> org, Off back = 0) {
+    const GlobalPtr<char> src = (GlobalPtr<char>)org + (off[i] - back);
+    if constexpr (kF32) {
+      using V = typename std::conditional<VEC, floatx4, floatx4u>::type;
+      const V q = *(GlobalPtr<V>)src;
+      r[i][0] = q[0]; r[i][1] = q[1]; r[i][2] = q[2]; r[i][3] = q[3];
+    } else {
+      // The four bytes; made floats at the store, where they are waited for.
+      r[i][0] = __builtin_bit_cast(float, *(GlobalPtr<uint32u>)src);
+    }
+  }
+  __device__ __forceinline__ void put(int i, int e, T x, bool in) {
+    if constexpr (kF32) {
+      r[i][e] = in ? x : 0.0f;
+    } else {
+      const uint32_t b = in ? static_cast<uint8_t>(x) : 0u;
+      const uint32_t w = e == 0 ? 0u : __builtin_bit_cast(uint32_t, r[i][0]);
+      r[i][0] = __builtin_bit_cast(float, w | (b << (8 * e)));
+    }
+  }
+  // Elements of vector i of a row of fewer than 4 (!VEC, row-contiguous).
+  __device__ __forceinline__ void load_few(int i, GlobalPtr<T> org, bool in_k) {
+    int o, k;
+    coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = in_k && o + e < avail;
+      put(i, e, org[in ? off[i] / kSize + o + e : 0], in);
+    }
+  }
+
+  // A whole stage in range: one load per vector, no masks.
+  __device__ __forceinline__ void load_full(GlobalPtr<T> org) {
+    if constexpr (!VEC && !KC) {
+      if (few) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) load_few(i, org, true);
+        return;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) load_vec(i, org);
+    if constexpr (SC) pend = true;
+  }
+
+  // Any stage (it starts before ke): k beyond ke reads as zero.
+  __device__ __forceinline__ void load(const T* __restrict__ X, int64_t ld, int64_t o0, int64_t k0,
+                                       int64_t ke) {
+    const GlobalPtr<T> org = ScalarBase(X + (KC ? o0 * ld + k0 : k0 * ld + o0));
+    const int64_t kvalid = ke - k0;
+    if (kvalid >= KT) {
+      load_full(org);
+      return;
+    }
+    if constexpr (SC) pend = false;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      int o, k;
+      coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
+      if constexpr (!VEC && KC) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in = k + e < kvalid;
+          put(i, e, org[off[i] / kSize + (in ? e : -k)], in);
+        }
+      } else {
+        const bool in = k < kvalid;  // VEC: a KC vector is wholly in or out (K % 4 == 0)
+        if constexpr (!VEC && !KC) {
+          if (few) {
+            load_few(i, org, in);
+            continue;
+          }
+        }
+        load_vec(i, org, in ? 0 : static_cast<Off>((KC ? k : k * ld) * kSize));
+        if constexpr (kF32) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (SC) r[i][e] = sc * r[i][e];
+            r[i][e] = in ? r[i][e] : 0.0f;
+          }
+        } else {
+          r[i][0] = in ? r[i][0] : 0.0f;
+        }
+      }
+    }
+  }
+
+  // Splits the stage into its parts and stores them.
+  __device__ __forceinline__ void store(__bf16* __restrict__ lds) const {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) store_vec(i, lds);
+  }
+  __device__ __forceinline__ void store_vec(int i, __bf16* __restrict__ lds) const {
+    {
+      int o, k;
+      coords(static_cast<int>(threadIdx.x) + i * NT, o, k);
+      __bf16* dst = KC ? lds + o * KT + KcChunk<KT>(o, k >> 3) * 8 + (k & 7)
+                       : lds + k * RcStride(MT) + o;
+      float q[4];
+      if constexpr (kF32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          q[e] = r[i][e];
+          if constexpr (SC) if (pend) q[e] = sc * q[e];
+        }
+        if constexpr (!VEC && !KC) {
+          if (avail < MT && !few) {  // this tile passes the row's end
+            if (shift[i] & 1) { q[0] = q[1]; q[1] = q[2]; q[2] = q[3]; q[3] = 0.0f; }
+            if (shift[i] & 2) { q[0] = q[2]; q[1] = q[3]; q[2] = q[3] = 0.0f; }
+            if (shift[i] >= 4) q[0] = q[1] = q[2] = q[3] = 0.0f;
+          }
+        }
+      } else {
+        uint32_t w = __builtin_bit_cast(uint32_t, r[i][0]);
+        if constexpr (!KC) {
+          if (avail < MT && !few) w = shift[i] >= 4 ? 0u : w >> (8 * shift[i]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = static_cast<float>(static_cast<int8_t>(w >> (8 * e)));
+      }
+      uint32_t lo[3], hi[3];
+      Split2(q[0], q[1], lo);
+      Split2(q[2], q[3], hi);
+#pragma unroll
+      for (int part = 0; part < kParts; ++part)
+        *reinterpret_cast<uint2*>(dst + part * kPlane) = make_uint2(lo[part], hi[part]);
     }
   }
 };
 
-// The 4 k values (8g + 4h + j, j = 0..3) of NB 32-wide fragments at o = w0 + 32i + r.
-template <int MT, int KT, bool KC, int NB>
-__device__ __forceinline__ void ReadFrags(const float* __restrict__ lds, int w0, int g, int h,
-                                          int r, float (&f)[NB][4]) {
+__device__ __forceinline__ bf16x4 ReadTr(const __bf16* p) {
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
+}
+
+// The parts of NB 32-wide fragments at o = w0 + 32i + r: k = 16g + 8h + 0..7.
+template <int MT, int KT, bool KC, int NB, int P>
+__device__ __forceinline__ void ReadFrags(const __bf16* __restrict__ lds, int w0, int g, int lane,
+                                          bf16x8 (&f)[NB][P]) {
+  constexpr int kPlane = PlaneElems<MT, KT, KC>();
+  const int h = lane >> 5;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int o = w0 + 32 * i + r;
     if constexpr (KC) {
-      const float4 q = *reinterpret_cast<const float4*>(lds + o * KcStride(KT) + g * KG + 4 * h);
-      f[i][0] = q.x; f[i][1] = q.y; f[i][2] = q.z; f[i][3] = q.w;
-    } else {
+      const int o = w0 + 32 * i + (lane & 31);
+      const __bf16* src = lds + o * KT + KcChunk<KT>(o, 2 * g + h) * 8;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) f[i][j] = lds[(g * KG + 4 * h + j) * RcStride(MT) + o];
+      for (int part = 0; part < P; ++part)
+        f[i][part] = *reinterpret_cast<const bf16x8*>(src + part * kPlane);
+    } else {
+      // A transposing read takes a [4 k][16 o] patch per 16 lanes, each lane
+      // naming 4 o of one k, and returns 4 k of one o.
+      const int k = KG * g + 8 * h + ((lane & 15) >> 2);
+      const int o = w0 + 32 * i + (lane & 16) + 4 * (lane & 3);
+#pragma unroll
+      for (int part = 0; part < P; ++part) {
+        const __bf16* src = lds + part * kPlane + k * RcStride(MT) + o;
+        f[i][part] = __builtin_shufflevector(ReadTr(src), ReadTr(src + 4 * RcStride(MT)), 0, 1, 2, 3,
+                                             4, 5, 6, 7);
+      }
     }
   }
 }
@@ -314,7 +563,7 @@ __device__ __forceinline__ uint32_t XcdLogical(uint32_t lin, uint32_t total) {
 // SCL: a Scale folded into the loads of A (1) or B (2), factor p.op_scale.
 // POST (with FUSED): the AddBias (+ activation) after the fused AddEW.
 template <int MT_M, int MT_N, int KT, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool B_I8,
-          bool VEC, bool SCHED, bool FUSED, bool LORA, int SCL = 0, bool POST = false>
+          bool VEC, bool FUSED, bool LORA, int SCL = 0, bool POST = false>
 __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32_t nslices) {
   static_assert(!POST || (FUSED && !LORA && !(MT_M == 256 && MT_N == 128)), "post-AddEW variants");
   using BT = typename std::conditional<B_I8, int8_t, float>::type;
@@ -323,10 +572,17 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   constexpr int BM = WM / 32, BN = WN / 32;
   static_assert(WM % 32 == 0 && WN % 32 == 0 && KT % KG == 0 && kSplitAlign % KT == 0,
                 "tile shape");
-  constexpr int TA = TileFloats<MT_M, KT, A_KC>(), TB = TileFloats<MT_N, KT, B_KC>();
-  __shared__ __align__(16) float smem[2 * (TA + TB)];
+  constexpr bool kVecB = VEC && !B_I8;
+  using StageA = Stage<MT_M, KT, A_KC, float, NT, VEC, SCL == 1>;
+  using StageB = Stage<MT_N, KT, B_KC, BT, NT, kVecB, SCL == 2>;
+  constexpr int TA = StageA::kElems, TB = StageB::kElems, PB = StageB::kParts;
+  __shared__ __align__(16) __bf16 smem[2 * (TA + TB)];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // What is one value per wavefront is kept in scalar registers (the
+  // divisions below run on the vector ALU): operand bases then cost no
+  // vector registers, and a load is a scalar base plus a 32-bit offset.
+  auto uniform = [](auto v) { return __builtin_amdgcn_readfirstlane(static_cast<int>(v)); };
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
   const int h = lane >> 5, r = lane & 31;
   const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
 
@@ -334,16 +590,16 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   const uint32_t tiles = static_cast<uint32_t>(p.tiles_m) * static_cast<uint32_t>(p.tiles_n);
   const uint32_t t_id = L % tiles;
   L /= tiles;
-  const int slice = static_cast<int>(L % nslices);
+  const int slice = uniform(L % nslices);
   const uint32_t z = L / nslices;
   const uint32_t grp = t_id / (kGroupRows * static_cast<uint32_t>(p.tiles_n));
   const uint32_t first = grp * kGroupRows;
   const uint32_t gm = std::min<uint32_t>(kGroupRows, static_cast<uint32_t>(p.tiles_m) - first);
   const uint32_t in_grp = t_id - grp * kGroupRows * static_cast<uint32_t>(p.tiles_n);
-  const int64_t tm = first + in_grp % gm, tn = in_grp / gm;
+  const int64_t tm = uniform(first + in_grp % gm), tn = uniform(in_grp / gm);
   const int64_t m0 = tm * MT_M, n0 = tn * MT_N;
   const uint32_t heads = static_cast<uint32_t>(p.heads);
-  const int64_t zb = z / heads, zh = z % heads;
+  const int64_t zb = uniform(z / heads), zh = uniform(z % heads);
 
   const float* A = static_cast<const float*>(p.A) + zb * p.a_sb + zh * p.a_sh;
   const BT* B = static_cast<const BT*>(p.B) + zb * p.b_sb + zh * p.b_sh;
@@ -367,48 +623,38 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     ke = std::min<int64_t>(p.K, kb + p.k_per_split);
   }
 
-  floatx16 acc[BM][BN];
+  floatx16 acc[BM][BN], sum[BM][BN];  // the current chunk's, and those before it
 #pragma unroll
   for (int i = 0; i < BM; ++i)
 #pragma unroll
     for (int j = 0; j < BN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v] = 0.0f;
 
-  constexpr bool kVecB = VEC && !B_I8;
-  using StageA = Stage<MT_M, KT, A_KC, float, NT, VEC, SCL == 1>;
-  using StageB = Stage<MT_N, KT, B_KC, BT, NT, kVecB, SCL == 2>;
   // Two register sets: stage s is loaded into set s % 2 two iterations
   // before it is computed, stored to LDS buffer s % 2 one iteration before.
   StageA sa0, sa1;
   StageB sb0, sb1;
 
-  // One stage's contraction out of LDS: 4 MFMAs per fragment group per
-  // (i, jj) block, the next group's fragments read while the current
-  // group's MFMAs run.
-  auto compute = [&](const float* __restrict__ as, const float* __restrict__ bs) {
-    float fa[2][BM][4], fb[2][BN][4];
-    ReadFrags<MT_M, KT, A_KC, BM>(as, wm0, 0, h, r, fa[0]);
-    ReadFrags<MT_N, KT, B_KC, BN>(bs, wn0, 0, h, r, fb[0]);
-#pragma unroll
-    for (int g = 0; g < KT / KG; ++g) {
-      const int c = g & 1;
-      if (g + 1 < KT / KG) {
-        ReadFrags<MT_M, KT, A_KC, BM>(as, wm0, g + 1, h, r, fa[c ^ 1]);
-        ReadFrags<MT_N, KT, B_KC, BN>(bs, wn0, g + 1, h, r, fb[c ^ 1]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < BM; ++i)
-#pragma unroll
-          for (int jj = 0; jj < BN; ++jj)
-            acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[c][i][j], fb[c][jj][j],
-                                                               acc[i][jj], 0, 0, 0);
-    }
-  };
   auto a_buf = [&](int i) { return smem + i * TA; };
   auto b_buf = [&](int i) { return smem + 2 * TA + i * TB; };
+  // One stage's contraction out of LDS. `fold`: the stage starts a chunk.
+  constexpr int kPerChunk = kChunk / KT;  // stages
+  auto compute = [&](const __bf16* __restrict__ as, const __bf16* __restrict__ bs, auto fold) {
+#pragma unroll
+    for (int g = 0; g < KT / KG; ++g) {
+      bf16x8 fa[BM][3], fb[BN][PB];
+      ReadFrags<MT_N, KT, B_KC, BN, PB>(bs, wn0, g, lane, fb);
+      ReadFrags<MT_M, KT, A_KC, BM, 3>(as, wm0, g, lane, fa);
+      if (decltype(fold)::value && g == 0) MfmaStep<true>(fa, fb, acc, sum);
+      else MfmaStep<false>(fa, fb, acc, sum);
+    }
+  };
+  auto compute_at = [&](int64_t s) {  // stage s from its buffer
+    const int cur = static_cast<int>(s & 1);
+    if (s % kPerChunk == 0) compute(a_buf(cur), b_buf(cur), std::true_type());
+    else compute(a_buf(cur), b_buf(cur), std::false_type());
+  };
 
   const int64_t span = ke > kb ? ke - kb : 0;
   const int64_t nfull = span / KT;
@@ -419,123 +665,116 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   const BT* b_org = B + (B_KC ? n0 * p.ldb + kb : kb * p.ldb + n0);
   // Loads stage s into a register set (any stage: k beyond ke reads zero).
   auto load_any = [&](StageA& xa, StageB& xb, int64_t s) {
-    xa.load(A, p.lda, m0, p.M, kb + s * KT, ke);
-    xb.load(B, p.ldb, n0, p.N, kb + s * KT, ke);
+    xa.load(A, p.lda, m0, kb + s * KT, ke);
+    xb.load(B, p.ldb, n0, kb + s * KT, ke);
   };
   // Loads stage s < nfull (wholly in range).
   auto load_full = [&](StageA& xa, StageB& xb, int64_t s) {
-    if constexpr (VEC) xa.load_full(a_org + s * a_step);
-    else xa.load(A, p.lda, m0, p.M, kb + s * KT, ke);
-    if constexpr (kVecB) xb.load_full(b_org + s * b_step);
-    else xb.load(B, p.ldb, n0, p.N, kb + s * KT, ke);
+    xa.load_full(ScalarBase(a_org + s * a_step));
+    xb.load_full(ScalarBase(b_org + s * b_step));
   };
   // Steady-state iteration on stage t (t + 2 < nfull): load stage t + 2 into
   // set `ld`, contract stage t, store stage t + 1 from set `st`. With VEC the
   // body is one basic block, scheduled as one interleave.
   auto steady = [&](StageA& lda_, StageB& ldb_, const StageA& sta, const StageB& stb,
-                    int64_t t, int cur) {
+                    int64_t t, int cur, auto fold) {
     load_full(lda_, ldb_, t + 2);
-    compute(a_buf(cur), b_buf(cur));
+    compute(a_buf(cur), b_buf(cur), fold);
     sta.store(a_buf(cur ^ 1));
     stb.store(b_buf(cur ^ 1));
-    if constexpr (SCHED) {
-      // Per MFMA: one LDS fragment read for a later group; global loads
-      // over the first half; the next stage's LDS writes over the second.
-      constexpr int kMfma = (KT / KG) * 4 * BM * BN;
-      constexpr int kVmem = StageA::kPer + StageB::kPer;
-      constexpr int kDsw = kVmem;
-      constexpr int kDsrGroup = (A_KC ? BM : 2 * BM) + (B_KC ? BN : 2 * BN);
-      __builtin_amdgcn_sched_group_barrier(0x100, kDsrGroup, 0);
-#pragma unroll
-      for (int i = 0; i < kMfma; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (i % 2 == 0 && i / 2 < kVmem) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        if (i >= kMfma / 2 && (i - kMfma / 2) % 2 == 0 && (i - kMfma / 2) / 2 < kDsw)
-          __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-      }
-    }
+    // One block per wavefront leaves too few MFMAs to hide the split under:
+    // there the scheduler's own order is the faster (64x64 tiles on
+    // 2048x512x1376: 27 us, interleaved 29; 128x64 tiles: 37, interleaved 33).
+    if constexpr (BM * BN > 1)
+      Interleave<(KT / KG) * BM * BN*(PB == 3 ? 6 : 3), StageA::kPer + StageB::kPer,
+                 BM * 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2)>();
     __syncthreads();
   };
 
-  // Early epilogue loads (kEarly: the 256x128 tile, one workgroup per CU,
-  // whose epilogue has no other workgroup's k loop to hide under; 128x256
-  // has no registers to spare for them in its NN group kernel): issued
-  // ahead of the last stage's MFMAs, so that their latency runs under them,
-  // into registers that take the dead k-loop staging registers' place. A
-  // fused AddEW's addend on a whole tile, or a LoRA epilogue's T and B'
-  // fragments, in one array `ep`: a work item takes at most one of them.
-  // Each addend load's address is a wave-uniform tile base plus a 32-bit
-  // byte offset (per-lane part + wave-uniform part), so loads in flight hold
-  // no 64-bit addresses. The values summed and their order are those of the
-  // loads after the k loop that the other tiles issue: the same bits.
-  // Measured alone on 8192x2048x2048, 8192x2048x5504 and 8192x5504x2048:
-  // the fused AddEW 0-6 us and the NT LoRA epilogue 30-86 us less per
-  // launch than with the loads after the k loop; the plain form unchanged.
-  constexpr bool kEarly = MT_M == 256 && MT_N == 128;
-  constexpr int kLoraG = 2;  // LoRA k groups held at once: rank <= 16
-  constexpr int kEp = std::max(BM * BN * 16, (BM + BN) * kLoraG * 4);
-  const bool lora_epi = LORA && p.lora_t;
-  const bool addend_early = kEarly && FUSED && !lora_epi && p.out && p.splits == 1 &&
-                            m0 + MT_M <= p.M && n0 + MT_N <= p.N &&
-                            MT_M * p.ldo * 4 < (int64_t{1} << 30);
-  float ep[kEp];
-  auto yv_at = [](int i, int j, int v) { return (i * BN + j) * 16 + v; };
-  auto ta_at = [](int i, int g, int q) { return (i * kLoraG + g) * 4 + q; };
-  auto tb_at = [](int j, int g, int q) { return BM * kLoraG * 4 + (j * kLoraG + g) * 4 + q; };
-  auto load_early = [&]() {
-    if constexpr (FUSED) {
-      if (addend_early) {
-        const char* y_base = reinterpret_cast<const char*>(p.addend + m0 * p.ldo + n0);
-        const uint32_t y_lane = static_cast<uint32_t>(((wm0 + 4 * h) * p.ldo + wn0 + r) * 4);
+  constexpr int kLoraK = 8;  // a lane's k of the LoRA product: 8h + 0..7, rank <= 16
+  // T's row and B's column entries of k = 8h + 0..7 (zero beyond the rank) of
+  // block row i / block column j. Unconditional loads (the half beyond the
+  // rank reads the other's and is zeroed), so that no branch splits the
+  // loads in flight.
+  auto load_lora_t = [&](int i, float* t) {
+    const int64_t row = std::min<int64_t>(m0 + wm0 + 32 * i + r, p.M - 1);
+    const bool in = 8 * h < p.lora_r;
+    const float4* src = reinterpret_cast<const float4*>(p.lora_t + row * p.lora_ldt + (in ? 8 * h : 0));
+    const float4 q0 = src[0], q1 = src[1];
+    const float q[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
-        for (int i = 0; i < BM; ++i)
+    for (int e = 0; e < kLoraK; ++e) t[e] = in ? q[e] : 0.0f;
+  };
+  auto load_lora_b = [&](int j, float* t) {
+    const int64_t col = std::min<int64_t>(n0 + wn0 + 32 * j + r, p.N - 1);
+    const bool in = 8 * h < p.lora_r;
 #pragma unroll
-          for (int j = 0; j < BN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-              const uint32_t uoff = static_cast<uint32_t>(
-                  ((32 * i + 8 * (v >> 2) + (v & 3)) * p.ldo + 32 * j) * 4);
-              ep[yv_at(i, j, v)] = *reinterpret_cast<const float*>(y_base + (y_lane + uoff));
-            }
-      }
-    }
-    if constexpr (LORA) {
-      if (lora_epi) {
-        // Unconditional loads (a k group beyond the rank reads group 0 and
-        // is zeroed), so that no branch splits the loads in flight.
-        const int ng = p.lora_r / KG;  // 1 or 2
-#pragma unroll
-        for (int i = 0; i < BM; ++i) {
-          const int64_t row = std::min<int64_t>(m0 + wm0 + 32 * i + r, p.M - 1);
-#pragma unroll
-          for (int g = 0; g < kLoraG; ++g) {
-            const int k0 = (g < ng ? g : 0) * KG + 4 * h;
-            const float4 q = *reinterpret_cast<const float4*>(p.lora_t + row * p.lora_ldt + k0);
-            ep[ta_at(i, g, 0)] = g < ng ? q.x : 0.0f;
-            ep[ta_at(i, g, 1)] = g < ng ? q.y : 0.0f;
-            ep[ta_at(i, g, 2)] = g < ng ? q.z : 0.0f;
-            ep[ta_at(i, g, 3)] = g < ng ? q.w : 0.0f;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < BN; ++j) {
-          const int64_t col = std::min<int64_t>(n0 + wn0 + 32 * j + r, p.N - 1);
-#pragma unroll
-          for (int g = 0; g < kLoraG; ++g)
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-              const int k = (g < ng ? g : 0) * KG + 4 * h + jj;
-              const float x = p.lora_b[k * p.lora_ldb + col];
-              ep[tb_at(j, g, jj)] = g < ng ? x : 0.0f;
-            }
-        }
-      }
+    for (int e = 0; e < kLoraK; ++e) {
+      const float x = p.lora_b[((in ? 8 * h : 0) + e) * p.lora_ldb + col];
+      t[e] = in ? x : 0.0f;
     }
   };
-
+  // kOneSet (the tiles of 64x64 wavefronts): their accumulators leave registers
+  // for one stage set only. Each vector of stage t + 1 is split and stored
+  // between the MFMAs of stage t, and its registers take stage t + 2's load at
+  // once.
+  constexpr bool kOneSet = BM * BN >= 4;
   int64_t t = 0;
-  if (ntiles > 0) {
+  if constexpr (kOneSet) {
+    constexpr int kVA = StageA::kPer, kV = kVA + StageB::kPer;
+    static_assert(KT == KG, "one fragment group per stage");
+    if (ntiles > 0) {
+      sa0.init(p.lda, m0, p.M);
+      sb0.init(p.ldb, n0, p.N);
+      if constexpr (SCL == 1) sa0.sc = p.op_scale;
+      if constexpr (SCL == 2) sb0.sc = p.op_scale;
+      load_any(sa0, sb0, 0);
+      sa0.store(a_buf(0));
+      sb0.store(b_buf(0));
+      if (ntiles > 1) load_any(sa0, sb0, 1);
+      __syncthreads();
+      auto body = [&](int64_t s, int cur, auto fold) {  // stage s, s + 2 whole
+        const GlobalPtr<float> a_next = ScalarBase(a_org + (s + 2) * a_step);
+        const GlobalPtr<BT> b_next = ScalarBase(b_org + (s + 2) * b_step);
+        bf16x8 fb[BN][PB];
+        ReadFrags<MT_N, KT, B_KC, BN, PB>(b_buf(cur), wn0, 0, lane, fb);
+#pragma unroll
+        for (int i = 0; i < BM; ++i) {
+          bf16x8 fa[1][3];
+          ReadFrags<MT_M, KT, A_KC, 1, 3>(a_buf(cur), wm0 + 32 * i, 0, lane, fa);
+          MfmaStep<decltype(fold)::value>(fa, fb, reinterpret_cast<floatx16(&)[1][BN]>(acc[i]),
+                                          reinterpret_cast<floatx16(&)[1][BN]>(sum[i]));
+#pragma unroll
+          for (int v = kV * i / BM; v < kV * (i + 1) / BM; ++v) {
+            if (v < kVA) {
+              sa0.store_vec(v, a_buf(cur ^ 1));
+              sa0.load_vec(v, a_next);
+            } else {
+              sb0.store_vec(v - kVA, b_buf(cur ^ 1));
+              sb0.load_vec(v - kVA, b_next);
+            }
+          }
+        }
+        Interleave<BM * BN*(PB == 3 ? 6 : 3), kV, 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2)>();
+        __syncthreads();
+      };
+      for (; t + kPerChunk + 1 < nfull; t += kPerChunk) {  // a chunk
+        body(t, 0, std::true_type());
+#pragma unroll
+        for (int u = 1; u < kPerChunk; ++u) body(t + u, u & 1, std::false_type());
+      }
+      for (; t < ntiles; ++t) {  // at most a chunk and two
+        compute_at(t);
+        if (t + 1 < ntiles) {
+          const int nxt = static_cast<int>(t & 1) ^ 1;
+          sa0.store(a_buf(nxt));
+          sb0.store(b_buf(nxt));
+          if (t + 2 < ntiles) load_any(sa0, sb0, t + 2);
+          __syncthreads();
+        }
+      }
+    }
+  } else if (ntiles > 0) {
     sa0.init(p.lda, m0, p.M);
     sb0.init(p.ldb, n0, p.N);
     sa1.init(p.lda, m0, p.M);
@@ -548,38 +787,25 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     sb0.store(b_buf(0));
     __syncthreads();
 
-    for (; t + 3 < nfull; t += 2) {
-      steady(sa0, sb0, sa1, sb1, t, 0);
-      steady(sa1, sb1, sa0, sb0, t + 1, 1);
-    }
-    // The remaining stages (fewer than four): masked loads where needed.
-    if constexpr (!kEarly) {
-      for (; t < ntiles; ++t) {
-        const int cur = static_cast<int>(t & 1);
-        if (t + 2 < ntiles) {
-          if (cur) load_any(sa1, sb1, t + 2);
-          else load_any(sa0, sb0, t + 2);
-        }
-        compute(a_buf(cur), b_buf(cur));
-        if (t + 1 < ntiles) {
-          if (cur) {
-            sa0.store(a_buf(0));
-            sb0.store(b_buf(0));
-          } else {
-            sa1.store(a_buf(1));
-            sb1.store(b_buf(1));
-          }
-          __syncthreads();
-        }
+    static_assert(kPerChunk % 2 == 0, "a chunk takes each register set alike often");
+    for (; t + kPerChunk + 1 < nfull; t += kPerChunk) {  // a chunk
+      steady(sa0, sb0, sa1, sb1, t, 0, std::true_type());
+      steady(sa1, sb1, sa0, sb0, t + 1, 1, std::false_type());
+#pragma unroll
+      for (int u = 2; u < kPerChunk; u += 2) {
+        steady(sa0, sb0, sa1, sb1, t + u, 0, std::false_type());
+        steady(sa1, sb1, sa0, sb0, t + u + 1, 1, std::false_type());
       }
-    } else {
-      for (; t + 1 < ntiles; ++t) {
-        const int cur = static_cast<int>(t & 1);
-        if (t + 2 < ntiles) {
-          if (cur) load_any(sa1, sb1, t + 2);
-          else load_any(sa0, sb0, t + 2);
-        }
-        compute(a_buf(cur), b_buf(cur));
+    }
+    // The remaining stages (at most a chunk and two): masked loads where needed.
+    for (; t < ntiles; ++t) {
+      const int cur = static_cast<int>(t & 1);
+      if (t + 2 < ntiles) {
+        if (cur) load_any(sa1, sb1, t + 2);
+        else load_any(sa0, sb0, t + 2);
+      }
+      compute_at(t);
+      if (t + 1 < ntiles) {
         if (cur) {
           sa0.store(a_buf(0));
           sb0.store(b_buf(0));
@@ -591,17 +817,40 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       }
     }
   }
-  if constexpr (kEarly) {
-    // The last stage, with the early epilogue loads in flight under its MFMAs
-    // (one program point for the loads, whether or not there is a stage).
-    // s_waitcnt vmcnt(0) (0x0F70: expcnt and lgkmcnt not waited on). No
-    // k-loop load is pending here; stated, it keeps the compiler from
-    // placing waits on the early loads inside the last stage's MFMAs.
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    load_early();
-    __builtin_amdgcn_sched_barrier(0);
-    if (ntiles > 0) compute(a_buf(static_cast<int>(t & 1)), b_buf(static_cast<int>(t & 1)));
-  }
+
+#pragma unroll
+  for (int i = 0; i < BM; ++i)
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v] + acc[i][j][v];
+
+  // Recompute: a suspect block's outputs by fp32 products, straight from
+  // memory (k pairs 16g + j, 16g + 8 + j). Decided per 32x32 block of the
+  // output, so that it does not depend on the tile config.
+#pragma unroll
+  for (int i = 0; i < BM; ++i)
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+      if (__builtin_expect(AnySuspect(acc[i][j]), false)) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+        const int64_t m = std::min<int64_t>(m0 + wm0 + 32 * i + r, p.M - 1);
+        const int64_t n = std::min<int64_t>(n0 + wn0 + 32 * j + r, p.N - 1);
+#pragma unroll 1
+        for (int64_t k0 = kb; k0 < ke; k0 += KG)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const bool in = k0 + 8 * h + e < ke;
+            const int64_t k = in ? k0 + 8 * h + e : k0;
+            float x = A[A_KC ? m * p.lda + k : k * p.lda + m];
+            float y = static_cast<float>(B[B_KC ? n * p.ldb + k : k * p.ldb + n]);
+            if constexpr (SCL == 1) x = p.op_scale * x;
+            if constexpr (SCL == 2) y = p.op_scale * y;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x : 0.0f, in ? y : 0.0f, acc[i][j],
+                                                             0, 0, 0);
+          }
+      }
 
   // A fused AddEW (GemmKArgs::out; FUSED instantiations, launched with one
   // slice and a plain epilogue). On a whole tile, each lane holds one base
@@ -610,65 +859,34 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   // are loaded first, all in flight together, then the sums are stored.
   // The value summed is the one the plain epilogue would store in C.
   if constexpr (LORA) if (p.lora_t) {
-    // u = T B' block by block (k = 8g + 4h + j for MFMA j of group g, as in
-    // the k loop above). Up to rank 16 every fragment of the wavefront's
-    // blocks is loaded at once, before any MFMA, so their latencies overlap;
-    // each block's outputs are stored right after its MFMAs (stores from one
-    // base pointer per lane, with no per-element bounds, measured 5% slower:
-    // the per-element form spreads them between the next block's MFMAs).
-    float ta[BM][kLoraG][4], tb[BN][kLoraG][4];
-    const int ng = p.lora_r / KG;
-    if constexpr (kEarly) {  // loaded ahead of the last stage
+    // u = T B' block by block, one step of the k loop above (its products,
+    // their order and its recomputation, so u has the bits of a tile GEMM).
+    // Every fragment of the wavefront's blocks is loaded at once, before any
+    // MFMA, so their latencies overlap; each block's outputs are stored right
+    // after its MFMAs (stores from one base pointer per lane, with no
+    // per-element bounds, measured 5% slower: the per-element form spreads
+    // them between the next block's MFMAs).
+    float tl[BM + BN][kLoraK];
 #pragma unroll
-      for (int i = 0; i < BM; ++i)
+    for (int i = 0; i < BM; ++i) load_lora_t(i, tl[i]);
 #pragma unroll
-        for (int g = 0; g < kLoraG; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) ta[i][g][q] = ep[ta_at(i, g, q)];
-    } else {
-#pragma unroll
-      for (int i = 0; i < BM; ++i) {
-        const int64_t row = std::min<int64_t>(m0 + wm0 + 32 * i + r, p.M - 1);
-#pragma unroll
-        for (int g = 0; g < kLoraG; ++g) {
-          const int k0 = g * KG + 4 * h;
-          float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-          if (g < ng) q = *reinterpret_cast<const float4*>(p.lora_t + row * p.lora_ldt + k0);
-          ta[i][g][0] = q.x; ta[i][g][1] = q.y; ta[i][g][2] = q.z; ta[i][g][3] = q.w;
-        }
-      }
-    }
-    if constexpr (kEarly) {
-#pragma unroll
-      for (int j = 0; j < BN; ++j)
-#pragma unroll
-        for (int g = 0; g < kLoraG; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) tb[j][g][q] = ep[tb_at(j, g, q)];
-    } else {
-#pragma unroll
-      for (int j = 0; j < BN; ++j) {
-        const int64_t col = std::min<int64_t>(n0 + wn0 + 32 * j + r, p.N - 1);
-#pragma unroll
-        for (int g = 0; g < kLoraG; ++g)
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj)
-            tb[j][g][jj] = g < ng ? p.lora_b[(g * KG + 4 * h + jj) * p.lora_ldb + col] : 0.0f;
-      }
-    }
+    for (int j = 0; j < BN; ++j) load_lora_b(j, tl[BM + j]);
 #pragma unroll
     for (int i = 0; i < BM; ++i)
 #pragma unroll
       for (int j = 0; j < BN; ++j) {
-        floatx16 u;
+        bf16x8 fa[1][3], fb[1][3];
+        Split8(tl[i], fa[0]);
+        Split8(tl[BM + j], fb[0]);
+        floatx16 ua[1][1] = {}, before[1][1] = {};
+        MfmaStep<true>(fa, fb, ua, before);
+        floatx16& u = ua[0][0];
+        if (__builtin_expect(AnySuspect(u), false)) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) u[v] = 0.0f;
+          for (int v = 0; v < 16; ++v) u[v] = 0.0f;
 #pragma unroll
-        for (int g = 0; g < kLoraG; ++g) {
-          if (g >= ng) break;
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj)
-            u = __builtin_amdgcn_mfma_f32_32x32x2f32(ta[i][g][jj], tb[j][g][jj], u, 0, 0, 0);
+          for (int e = 0; e < kLoraK; ++e)
+            u = __builtin_amdgcn_mfma_f32_32x32x2f32(tl[i][e], tl[BM + j][e], u, 0, 0, 0);
         }
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
@@ -682,27 +900,6 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       }
     return;
   }
-  if constexpr (FUSED && kEarly) {
-    if (addend_early) {
-      const int64_t lm = m0 + wm0 + 4 * h, ln = n0 + wn0 + r;
-      float* oa = p.out + lm * p.ldo + ln;
-      float* ca = C + lm * p.ldc + ln;
-#pragma unroll
-      for (int i = 0; i < BM; ++i)
-#pragma unroll
-        for (int j = 0; j < BN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int64_t row = 32 * i + 8 * (v >> 2) + (v & 3);
-            const float val = dev_act(p.act, p.alpha * acc[i][j][v]);
-            const float sv = p.out_scaled ? p.out_scale * val : val;
-            if (p.write_c) ca[row * p.ldc + 32 * j] = p.c_scaled ? sv : val;
-            const float y = ep[yv_at(i, j, v)];
-            oa[row * p.ldo + 32 * j] = p.addend_first ? y + sv : sv + y;
-          }
-      return;
-    }
-  }
   if constexpr (FUSED) {
     if (p.out && p.splits == 1 && m0 + MT_M <= p.M && n0 + MT_N <= p.N &&
         (!POST || MT_M * p.ldo * 4 < (int64_t{1} << 30))) {
@@ -710,7 +907,6 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       const float* ya = p.addend + lm * p.ldo + ln;
       float* oa = p.out + lm * p.ldo + ln;
       float* ca = C + lm * p.ldc + ln;
-      float yv[BM][BN][16];
       float pb[BN];  // POST: the AddBias values of the lane's columns
 #pragma unroll
       for (int j = 0; j < BN; ++j) pb[j] = POST ? p.pbias[ln + 32 * j] : 0.0f;
@@ -719,6 +915,7 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       char* post_h = POST && p.hout ? reinterpret_cast<char*>(p.hout + tile0) : nullptr;
       char* post_g = POST && p.gout ? reinterpret_cast<char*>(p.gout + tile0) : nullptr;
       const uint32_t post_lane = static_cast<uint32_t>(((lm - m0) * p.ldo + (ln - n0)) * 4);
+      float yv[BM][BN][16];
 #pragma unroll
       for (int i = 0; i < BM; ++i)
 #pragma unroll
@@ -816,12 +1013,12 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
 }
 
 template <int MT_M, int MT_N, int KT, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool B_I8,
-          bool VEC, bool SCHED, bool FUSED, bool LORA = false, int SCL = 0, bool POST = false>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_mfma_kernel(GemmKArgs p) {
+          bool VEC, bool FUSED, bool LORA = false, int SCL = 0, bool POST = false>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, MinWaves(MT_M, MT_N)) void gemm_mfma_kernel(GemmKArgs p) {
   const uint32_t tiles = static_cast<uint32_t>(p.tiles_m) * static_cast<uint32_t>(p.tiles_n);
   const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
   const uint32_t L = XcdLogical(lin, tiles * gridDim.y * gridDim.z);
-  gemm_tile<MT_M, MT_N, KT, WAVES_M, WAVES_N, A_KC, B_KC, B_I8, VEC, SCHED, FUSED, LORA, SCL, POST>(
+  gemm_tile<MT_M, MT_N, KT, WAVES_M, WAVES_N, A_KC, B_KC, B_I8, VEC, FUSED, LORA, SCL, POST>(
       p, L, gridDim.y);
 }
 
@@ -839,42 +1036,51 @@ struct GemmGroupArgs {
 };
 
 template <int MT_M, int MT_N, int KT, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool LORA>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_group_kernel(GemmGroupArgs g) {
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, MinWaves(MT_M, MT_N)) void gemm_group_kernel(GemmGroupArgs g) {
   const uint32_t total = g.wg_end[g.count - 1];
   uint32_t L = XcdLogical(blockIdx.x, total);
   uint32_t j = 0;
   while (j + 1 < g.count && L >= g.wg_end[j]) ++j;
   if (j > 0) L -= g.wg_end[j - 1];
-  gemm_tile<MT_M, MT_N, KT, WAVES_M, WAVES_N, A_KC, B_KC, false, true, true, true, LORA>(g.m[j], L, 1);
+  gemm_tile<MT_M, MT_N, KT, WAVES_M, WAVES_N, A_KC, B_KC, false, true, true, LORA>(g.m[j], L, 1);
 }
 
-// Launches config `cfg` of one operand-layout variant. The element-load
-// form (!VEC) exists only for the small tile; the host plans it as such.
-template <bool A_KC, bool B_KC, bool B_I8, bool VEC, bool SCHED = false, bool FUSED = false>
+// The tile config the general form (!VEC: any extent, stride and alignment;
+// int8) runs plan config `cfg` on: it exists for one large tile, whose 32x64 wavefronts leave it the
+// registers, and the small one.
+inline constexpr int GeneralCfg(int cfg) {
+  return cfg <= 3 ? 1 : kCfgSmall;
+}
+
+// Launches config `cfg` of one operand-layout variant.
+template <bool A_KC, bool B_KC, bool B_I8, bool VEC, bool FUSED = false>
 void LaunchVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) {
   const dim3 block(kCfgs[cfg].threads);
 #define SEEML_GEMM_CASE(I, MM, NN, KK, WM_, WN_)                                                \
   case I:                                                                                     \
-    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, B_I8, VEC, SCHED, FUSED>), grid, \
+    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, B_I8, VEC, FUSED>), grid, \
                        block, 0, s, a);                                                       \
     break;
   if constexpr (!VEC) {
-    hipLaunchKernelGGL((gemm_mfma_kernel<64, 64, 32, 2, 2, A_KC, B_KC, B_I8, false, false, false>), grid,
-                       dim3(kCfgs[kCfgSmall].threads), 0, s, a);
+    switch (GeneralCfg(cfg)) {
+      SEEML_GEMM_CASE(1, 128, 128, 16, 4, 2)
+      default:
+      SEEML_GEMM_CASE(5, 64, 64, 32, 2, 2)
+    }
   } else {
     switch (cfg) {
-      SEEML_GEMM_CASE(0, 128, 128, 32, 2, 2)
-      SEEML_GEMM_CASE(1, 128, 128, 32, 4, 2)
-      SEEML_GEMM_CASE(2, 256, 128, 32, 4, 2)
-      SEEML_GEMM_CASE(3, 128, 256, 32, 2, 4)
+      SEEML_GEMM_CASE(0, 128, 128, 16, 2, 2)
+      SEEML_GEMM_CASE(1, 128, 128, 16, 4, 2)
+      SEEML_GEMM_CASE(2, 256, 128, 16, 4, 2)
+      SEEML_GEMM_CASE(3, 128, 256, 16, 2, 4)
       SEEML_GEMM_CASE(4, 128, 64, 32, 2, 2)
       SEEML_GEMM_CASE(5, 64, 64, 32, 2, 2)
       SEEML_GEMM_CASE(6, 128, 32, 32, 4, 1)
       SEEML_GEMM_CASE(7, 32, 128, 32, 1, 4)
       SEEML_GEMM_CASE(8, 64, 128, 32, 2, 2)
       SEEML_GEMM_CASE(9, 128, 64, 32, 4, 1)
-      SEEML_GEMM_CASE(10, 128, 128, 16, 2, 2)
-      default:
+      SEEML_GEMM_CASE(10, 64, 64, 16, 2, 2)
+        default:
       SEEML_GEMM_CASE(11, 64, 128, 16, 2, 2)
     }
   }
@@ -889,12 +1095,12 @@ template <bool A_KC, bool B_KC>
 bool LaunchLoraVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) {
 #define SEEML_LORA_CASE(I, MM, NN, KK, WM_, WN_)                                                       \
   case I:                                                                                            \
-    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, true, true, true>), \
+    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, true, true>), \
                        grid, dim3(kCfgs[I].threads), 0, s, a);                                       \
     return true;
   switch (cfg) {
-    SEEML_LORA_CASE(0, 128, 128, 32, 2, 2)
-    SEEML_LORA_CASE(2, 256, 128, 32, 4, 2)
+    SEEML_LORA_CASE(0, 128, 128, 16, 2, 2)
+    SEEML_LORA_CASE(2, 256, 128, 16, 4, 2)
     SEEML_LORA_CASE(4, 128, 64, 32, 2, 2)
     SEEML_LORA_CASE(5, 64, 64, 32, 2, 2)
     SEEML_LORA_CASE(8, 64, 128, 32, 2, 2)
@@ -919,13 +1125,13 @@ bool LaunchGroupVariant(int cfg, dim3 grid, hipStream_t s, const GemmGroupArgs& 
                        dim3(kCfgs[I].threads), 0, s, g);                                         \
     return true;
   switch (cfg) {
-    SEEML_GROUP_CASE(0, 128, 128, 32, 2, 2)
-    SEEML_GROUP_CASE(2, 256, 128, 32, 4, 2)
+    SEEML_GROUP_CASE(0, 128, 128, 16, 2, 2)
+    SEEML_GROUP_CASE(2, 256, 128, 16, 4, 2)
     SEEML_GROUP_CASE(4, 128, 64, 32, 2, 2)
     SEEML_GROUP_CASE(5, 64, 64, 32, 2, 2)
     SEEML_GROUP_CASE(8, 64, 128, 32, 2, 2)
-    SEEML_GROUP_CASE(1, 128, 128, 32, 4, 2)
-    SEEML_GROUP_CASE(3, 128, 256, 32, 2, 4)
+    SEEML_GROUP_CASE(1, 128, 128, 16, 4, 2)
+    SEEML_GROUP_CASE(3, 128, 256, 16, 2, 4)
     SEEML_GROUP_CASE(9, 128, 64, 32, 4, 1)
     default:
       return false;
@@ -942,7 +1148,7 @@ template <bool A_KC, bool B_KC, int SCL>
 bool LaunchScaledVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) {
 #define SEEML_SCALED_CASE(I, MM, NN, KK, WM_, WN_)                                                     \
   case I:                                                                                            \
-    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, true, false, false, \
+    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, false, false, \
                                          SCL>),                                                      \
                        grid, dim3(kCfgs[I].threads), 0, s, a);                                       \
     return true;
@@ -951,7 +1157,7 @@ bool LaunchScaledVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) 
     SEEML_SCALED_CASE(5, 64, 64, 32, 2, 2)
     SEEML_SCALED_CASE(8, 64, 128, 32, 2, 2)
     SEEML_SCALED_CASE(9, 128, 64, 32, 4, 1)
-    SEEML_SCALED_CASE(10, 128, 128, 16, 2, 2)
+    SEEML_SCALED_CASE(10, 64, 64, 16, 2, 2)
     SEEML_SCALED_CASE(11, 64, 128, 16, 2, 2)
     default:
       return false;
@@ -966,7 +1172,7 @@ template <bool A_KC, bool B_KC>
 bool LaunchPostVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) {
 #define SEEML_POST_CASE(I, MM, NN, KK, WM_, WN_)                                                      \
   case I:                                                                                            \
-    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, true, true, false, \
+    hipLaunchKernelGGL((gemm_mfma_kernel<MM, NN, KK, WM_, WN_, A_KC, B_KC, false, true, true, false, \
                                          0, true>),                                                  \
                        grid, dim3(kCfgs[I].threads), 0, s, a);                                       \
     return true;
@@ -975,7 +1181,7 @@ bool LaunchPostVariant(int cfg, dim3 grid, hipStream_t s, const GemmKArgs& a) {
     SEEML_POST_CASE(5, 64, 64, 32, 2, 2)
     SEEML_POST_CASE(8, 64, 128, 32, 2, 2)
     SEEML_POST_CASE(9, 128, 64, 32, 4, 1)
-    SEEML_POST_CASE(10, 128, 128, 16, 2, 2)
+    SEEML_POST_CASE(10, 64, 64, 16, 2, 2)
     SEEML_POST_CASE(11, 64, 128, 16, 2, 2)
     default:
       return false;

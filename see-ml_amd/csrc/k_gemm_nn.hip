@@ -9,8 +9,8 @@ void LaunchNN(int cfg, bool vec, dim3 grid, hipStream_t s, const GemmKArgs& a) {
     (void)LaunchLoraVariant<true, false>(cfg, grid, s, a);
     return;
   }
-  if (vec && a.out && a.splits == 1) LaunchVariant<true, false, false, true, true, true>(cfg, grid, s, a);
-  else if (vec) LaunchVariant<true, false, false, true, true>(cfg, grid, s, a);
+  if (vec && a.out && a.splits == 1) LaunchVariant<true, false, false, true, true>(cfg, grid, s, a);
+  else if (vec) LaunchVariant<true, false, false, true>(cfg, grid, s, a);
   else LaunchVariant<true, false, false, false>(cfg, grid, s, a);
 }
 

@@ -9,8 +9,8 @@ void LaunchNT(int cfg, bool vec, dim3 grid, hipStream_t s, const GemmKArgs& a) {
     (void)LaunchLoraVariant<true, true>(cfg, grid, s, a);
     return;
   }
-  if (vec && a.out && a.splits == 1) LaunchVariant<true, true, false, true, true, true>(cfg, grid, s, a);
-  else if (vec) LaunchVariant<true, true, false, true, true>(cfg, grid, s, a);
+  if (vec && a.out && a.splits == 1) LaunchVariant<true, true, false, true, true>(cfg, grid, s, a);
+  else if (vec) LaunchVariant<true, true, false, true>(cfg, grid, s, a);
   else LaunchVariant<true, true, false, false>(cfg, grid, s, a);
 }
 

@@ -5,8 +5,8 @@ namespace seeml_hip {
 namespace gemm {
 
 void LaunchTN(int cfg, bool vec, dim3 grid, hipStream_t s, const GemmKArgs& a) {
-  if (vec && a.out && a.splits == 1) LaunchVariant<false, false, false, true, true, true>(cfg, grid, s, a);
-  else if (vec) LaunchVariant<false, false, false, true, true>(cfg, grid, s, a);
+  if (vec && a.out && a.splits == 1) LaunchVariant<false, false, false, true, true>(cfg, grid, s, a);
+  else if (vec) LaunchVariant<false, false, false, true>(cfg, grid, s, a);
   else LaunchVariant<false, false, false, false>(cfg, grid, s, a);
 }
 

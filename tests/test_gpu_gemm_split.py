@@ -1,0 +1,127 @@
+"""The tile GEMMs' bf16-split products at the sizes, alignments and values
+where they can go wrong: partial tiles and stages, rows of fewer than four
+elements, element-aligned operands (the general load form), int8 weights, and
+values the split cannot hold (recomputed in fp32).
+
+Tolerance: the operands are held exactly and the accumulator adds at most 24
+rounded terms per 16 k within a chunk of 64, then one per chunk; each rounding
+is at most 2^-24 of a partial sum, so the relative 2-norm error of a random
+product stays below sqrt(24 * 4 + K / 64) * 2^-24 (6e-7 at K = 64, 8e-7 at
+K = 4096)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+f32 = np.float32
+LAYOUTS = ("gemm_nn", "gemm_nt", "gemm_tn")
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from seeml_amd import _lib
+    return torch, _lib.lib()
+
+
+def device(torch, a, shift):
+    """`a` on the GPU, `shift` elements past a 16-byte boundary."""
+    buf = torch.zeros(a.size + 8, dtype=torch.from_numpy(a[:1]).dtype, device="cuda:0")
+    view = buf[shift:shift + a.size]
+    view.copy_(torch.from_numpy(a))
+    return view
+
+
+def call(gpu, name, *args):
+    torch, L = gpu
+    rc = getattr(L, "seeml_hip_" + name)(
+        *[a.data_ptr() if hasattr(a, "data_ptr") else a for a in args],
+        torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0, L.seeml_hip_kernel_error().decode()
+
+
+def bound(K):
+    return np.sqrt(96 + K / 64) * 2.0 ** -24
+
+
+SIZES = [(1, 1, 1), (2, 3, 5), (3, 2, 64), (5, 130, 3), (130, 3, 17), (63, 65, 15), (65, 63, 33),
+         (129, 131, 127), (257, 129, 66), (255, 259, 1027), (1000, 1531, 770)]
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_any_extent_and_alignment(gpu, M, N, K, shift):
+    torch, _ = gpu
+    r = np.random.default_rng([M, N, K])
+    A, B = r.standard_normal((M, K), dtype=f32), r.standard_normal((K, N), dtype=f32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    for layout, name in enumerate(LAYOUTS):
+        a = device(torch, np.ascontiguousarray(A.T if layout == 2 else A).ravel(), shift)
+        b = device(torch, np.ascontiguousarray(B.T if layout == 1 else B).ravel(), shift)
+        out = torch.full((M * N + 4,), 7.0, device="cuda:0")
+        call(gpu, name, a, b, out[:M * N], M, N, K, *((None, 0) if layout == 0 else ()))
+        got = out.cpu().numpy()
+        assert np.all(got[M * N:] == 7.0)
+        d = got[:M * N].reshape(M, N) - want
+        assert np.linalg.norm(d) <= bound(K) * np.linalg.norm(np.abs(A).astype(np.float64)
+                                                              @ np.abs(B)), name
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 5, 7), (65, 67, 33), (130, 258, 1030), (2048, 2048, 256)])
+def test_int8_weights(gpu, M, N, K):
+    torch, _ = gpu
+    r = np.random.default_rng([M, N, K, 8])
+    A = r.standard_normal((M, K), dtype=f32)
+    B = r.integers(-128, 128, (K, N)).astype(np.int8)
+    want = 0.01 * (A.astype(np.float64) @ B.astype(np.float64))
+    size = 0.01 * np.linalg.norm(np.abs(A).astype(np.float64) @ np.abs(B.astype(np.float64)))
+    a = device(torch, A.ravel(), 0)
+    for name, b in (("gemm_nn_q8", B), ("gemm_nt_q8", np.ascontiguousarray(B.T))):
+        out = torch.empty(M * N, device="cuda:0")
+        call(gpu, name, a, device(torch, b.ravel(), 3), out, M, N, K, float(f32(0.01)),
+             *((0,) if name == "gemm_nn_q8" else ()))
+        # one more rounding: the scale, itself 0.01 to 2^-24
+        assert np.linalg.norm(out.cpu().numpy().reshape(M, N) - want) <= (bound(K) + 2.0 ** -23) * size
+
+
+@pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny"])
+def test_values_the_split_cannot_hold(gpu, kind):
+    """One row carries them; its block is recomputed in fp32 and every other
+    output keeps its bits, on every tile config and with split-K."""
+    torch, L = gpu
+    M, N, K = 200, 136, 200
+    r = np.random.default_rng(9)
+    A, B = r.standard_normal((M, K), dtype=f32), r.standard_normal((K, N), dtype=f32)
+    clean = torch.empty(M * N, device="cuda:0")
+    b = device(torch, B.ravel(), 0)
+    call(gpu, "gemm_forced", 0, device(torch, A.ravel(), 0), b, clean, M, N, K, 0, 1)
+    bad = A.copy()
+    if kind == "tiny":  # results around 1e-36, operand parts below 2^-133
+        bad[70] *= f32(1e-36)
+    else:
+        bad[70, 33] = {"inf": np.inf, "nan": np.nan, "huge": 3.4e38}[kind]
+        B[33] *= f32(1e-3)
+        b = device(torch, B.ravel(), 0)
+        call(gpu, "gemm_forced", 0, device(torch, A.ravel(), 0), b, clean, M, N, K, 0, 1)
+    with np.errstate(all="ignore"):
+        want = (bad[70].astype(np.float64) @ B.astype(np.float64))
+    first = None
+    for cfg in range(L.seeml_hip_gemm_config_count() - 1):
+        out = torch.empty(M * N, device="cuda:0")
+        call(gpu, "gemm_forced", 0, device(torch, bad.ravel(), 0), b, out, M, N, K, cfg, 1)
+        got = out.cpu().numpy().reshape(M, N)
+        if kind == "nan":
+            assert np.all(np.isnan(got[70]))
+        elif kind == "inf":
+            assert np.array_equal(got[70], np.sign(B[33]) * f32(np.inf))
+        else:
+            assert np.linalg.norm(got[70] - want) <= 1e-6 * np.linalg.norm(want)
+        # rows outside the recomputed blocks (64..95) are untouched
+        keep = np.r_[0:64, 96:M]
+        assert np.array_equal(got[keep].view(np.uint32),
+                              clean.cpu().numpy().reshape(M, N)[keep].view(np.uint32)), cfg
+        first = got if first is None else first
+        assert np.array_equal(got.view(np.uint32), first.view(np.uint32)) or kind == "nan", cfg
