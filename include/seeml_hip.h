@@ -127,7 +127,7 @@ uint64_t seeml_hip_workspace_bytes(const seeml_hip_engine* e);
 /* GEMM tile autotuning (compiler/backend/tuner/bandit.cc:14-53,
  * autotuner.cc:21-80 retargeted to GPU tiles): for every distinct GEMM shape
  * of the train program, a deterministic UCB1 bandit over tile arms, reward =
- * measured fraction of fp32 MFMA peak. Every arm keeps the summation order
+ * measured fraction of the matrix cores' peak. Every arm keeps the summation order
  * the shape fixes (the split-K count, or the skinny kernels' order): arms
  * differ only in tile config or column split (whole rounds of 256x128 tiles,
  * the rest on smaller tiles), which change no bits, so an autotuned run has

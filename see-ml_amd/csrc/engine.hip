@@ -73,7 +73,9 @@ bool IsGemmOp(uint16_t op) {
 // standalone timings that close do not rank the tiles inside the step's
 // graph, so near-ties keep the planner's hint (arm 0) or the earlier config.
 constexpr double kAutotuneTileTolerance = 0.015;
-constexpr double kPeakFp32MfmaFlops = 157.3e12;  // MI355X dense fp32 matrix peak
+// Peak rate of fp32 products as the tile GEMMs form them: six bf16 products
+// each, on matrix cores of 2.5 PFLOP/s dense.
+constexpr double kPeakGemmFlops = 2516.6e12 / 6;
 
 class Ucb1 {
  public:
@@ -3054,7 +3056,7 @@ class Engine {
         (void)hipEventSynchronize(t1);
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, t0, t1);
-        bandit.Update(arm, ms > 0.0f ? flops / (ms * 1e-3) / kPeakFp32MfmaFlops : 0.0);
+        bandit.Update(arm, ms > 0.0f ? flops / (ms * 1e-3) / kPeakGemmFlops : 0.0);
       }
       const int best = arms[bandit.Best(kAutotuneTileTolerance)];
       picked[key] = best;
@@ -3206,7 +3208,7 @@ class Engine {
         if (ms > 0.0f) reps[a] = std::clamp(static_cast<int>(0.2f / ms), 1, 16);
       }
       if (!result) break;
-      // Rewards are the fraction of fp32 MFMA peak (UCB1's [0, 1] scale);
+      // Rewards are the fraction of the GEMMs' peak (UCB1's [0, 1] scale);
       // every arm is pulled at least twice.
       Ucb1 bandit(arms.size());
       const int trials = std::max<int>(budget, 2 * static_cast<int>(arms.size()));
@@ -3221,7 +3223,7 @@ class Engine {
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, t0, t1);
         ms /= static_cast<float>(reps[arm]);
-        bandit.Update(arm, ms > 0.0f ? flops / (ms * 1e-3) / kPeakFp32MfmaFlops : 0.0);
+        bandit.Update(arm, ms > 0.0f ? flops / (ms * 1e-3) / kPeakGemmFlops : 0.0);
       }
       if (!result) break;
       const GemmPlan best = arms[bandit.Best(kAutotuneTileTolerance)];

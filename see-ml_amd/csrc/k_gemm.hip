@@ -1,4 +1,4 @@
-// k_gemm.hip — host side of the fp32 MFMA GEMM engine: tile planning,
+// k_gemm.hip — host side of the matrix-core GEMM engine (fp32): tile planning,
 // split-K, launch-shape checks and the split-K reduction kernel. The kernel
 // template itself is in k_gemm_kernel.h (design notes there), instantiated
 // per operand layout in k_gemm_{nn,nt,tn,q8}.hip.

@@ -1,4 +1,4 @@
-// k_gemm_kernel.h — the fp32 MFMA GEMM kernel template for gfx950 (device code
+// k_gemm_kernel.h — the fp32 GEMM kernel template on gfx950 matrix cores (device code
 // shared by the per-layout instantiation units k_gemm_{nn,nt,tn,q8}.hip; host
 // planning and launch live in k_gemm.hip).
 //
