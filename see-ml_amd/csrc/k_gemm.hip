@@ -102,8 +102,9 @@ int TileFor(const GemmDesc& d) {
 // cover the chip twice with 64x64 or 128x128 tiles, each at least 128 deep.
 // Elsewhere a slice costs a pass over the output and a launch (about 5 us),
 // against about 0.6 us per 32 of depth that a lone workgroup takes: slices of
-// 1024 where the output leaves CUs idle (600x1024x1024 takes 24 us in one
-// slice, 600x1024x4096 82 us in one and 48 in four), otherwise none.
+// 1024, no more than two 128x128 tiles' worth per CU, where the output leaves
+// CUs idle (600x1024x1024 takes 24 us in one slice, 600x1024x4096 82 us in one
+// and 48 in four), otherwise none.
 int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
   if (d.batch != 1 || d.causal != Causal::kNone || d.K < 256) return 1;
   const int64_t big = CeilDiv(d.M, 128) * CeilDiv(d.N, 128), mid = CeilDiv(d.M, 64) * CeilDiv(d.N, 64);
@@ -113,7 +114,7 @@ int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
             : d.M <= 32 && d.N > 32 ? CeilDiv(d.N, 128)
             : big >= 512 || (mid < 256 && d.M > 64 && d.N > 64) ? big : mid;
   } else if (mid < 256) {
-    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(d.K / 1024, 64)));
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(d.K / 1024, CeilDiv(512, big))));
   } else {
     return 1;
   }
