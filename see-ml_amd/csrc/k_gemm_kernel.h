@@ -43,17 +43,23 @@
 // log-normal operands 6.6e-7 | 1.3e-7 (without the second accumulator 7.0e-7
 // on the second, and gradients summed over 2048 rows were further off than
 // with the fp32 MFMA). An int8 operand is one bf16 part: three products.
-// Measured: NT 8192x2048x5504 1330 -> 890 us, 8192x5504x2048 1340 -> 975 us,
-// 190-208 TFLOP/s of fp32 products where 157 was the fp32 MFMA's peak. What
+// Measured: NT 8192x2048x5504 1330 -> 854 us, 8192x5504x2048 1334 -> 921 us,
+// 200-216 TFLOP/s of fp32 products where 157 was the fp32 MFMA's peak. What
 // bounds it now is power: the matrix cores are 76% busy at 1.74 GHz (2.4 with
 // little to do), and a loop of bf16 MFMAs alone on random bits runs at the
 // clock that makes 300.
 //
-// What the split cannot hold (an infinity or NaN, a value that rounds past
-// bf16's largest, a result so small that parts below 2^-133 matter) shows in
-// the accumulators: non-finite, or nonzero below 2^-100. A wavefront that
-// finds one in a 32x32 block computes that block again with the fp32 MFMA,
-// straight from memory (Recompute below), so non-finites propagate as fp32 products do.
+// Range. fp32 operands are scaled by 2^24 (kOpScale, exact) before the split,
+// and the sums by 2^-48 after it (2^-24 with an int8 operand): the smallest
+// subnormal becomes 2^-125, so every part of every value is zero or a normal
+// bf16 number, and what underflows among the products is below 2^-174 of the
+// true scale, under a K-th of fp32's smallest subnormal for any K here.
+// Unscaled, values under 2^-110 lost their low parts and those under 2^-134
+// vanished, which a large other factor could lift to any size. Infinities and
+// NaN, operands of 2^103 and more and sums of 2^80 and more do not survive the
+// scaled split and show as non-finite accumulators: a wavefront that finds one
+// in a 32x32 block computes that block again with the fp32 MFMA, straight
+// from memory (Recompute below), so non-finites propagate as fp32 products do.
 //
 // k assignment: half-wavefront h supplies k = 16g + 8h + 0..7 of the group
 // g of 16, for A and B alike. The split happens once per element and
@@ -129,10 +135,12 @@ __device__ __forceinline__ GlobalPtr<T> ScalarBase(const T* p) {
   return q;
 }
 
-// x as three bf16 parts, x = part 0 + part 1 + part 2 exactly for every
-// finite x of at most bf16's range and at least 2^-110 (below, part 2 loses
-// what lies under 2^-133). Packed: part i of (x0, x1) in p[i].
+// 2^24 x as three bf16 parts, 2^24 x = part 0 + part 1 + part 2 exactly for
+// every |x| below 2^103. Packed: part i of (x0, x1) in p[i].
+constexpr float kOpScale = 0x1p24f, kOpUnscale = 0x1p-24f;
 __device__ __forceinline__ void Split2(float x0, float x1, uint32_t (&p)[3]) {
+  x0 *= kOpScale;
+  x1 *= kOpScale;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const bf16x2 h = __builtin_convertvector((floatx2){x0, x1}, bf16x2);
@@ -143,6 +151,11 @@ __device__ __forceinline__ void Split2(float x0, float x1, uint32_t (&p)[3]) {
       x1 -= __builtin_bit_cast(float, p[i] & 0xFFFF0000u);
     }
   }
+}
+
+// A pair of int8 values, each one part, unscaled.
+__device__ __forceinline__ uint32_t Exact2(float x0, float x1) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x0, x1}, bf16x2));
 }
 
 // The parts of a lane's 8 consecutive k.
@@ -188,36 +201,33 @@ __device__ __forceinline__ void MfmaStep(const bf16x8 (&fa)[BM][3], const bf16x8
 }
 
 // The issue order of one stage: kFirst fragment reads, then after each of the
-// kMfma MFMAs its share of the VALU operations that split kVecs vectors (22
-// each and their addresses), one LDS read, one LDS write and one global load.
-// Left to itself the scheduler issues the MFMAs first and the split after
-// them, so that a wavefront alone on its SIMD takes the sum of the two.
-template <int kMfma, int kVecs, int kFirst>
+// kMfma MFMAs its share of the VALU operations that split kVecs vectors
+// (kSplitOps each; 26 are the split, the rest room for addresses), LDS reads,
+// an LDS write and, unless they are issued ahead of it all (kAhead), a global
+// load. Left to itself the scheduler issues the MFMAs first and the split
+// after them, so that a wavefront alone on its SIMD takes the sum of the two.
+template <int kMfma, int kVecs, int kFirst, int kSplitOps, bool kAhead>
 __device__ __forceinline__ void Interleave() {
+  constexpr int kOps = (kSplitOps * kVecs + kMfma - 1) / kMfma;
   __builtin_amdgcn_sched_group_barrier(0x100, kFirst, 0);
 #pragma unroll
   for (int q = 0; q < kMfma; ++q) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x002, (24 * kVecs + kMfma - 1) / kMfma, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    if constexpr (kAhead) __builtin_amdgcn_sched_group_barrier(0x100, (kFirst + 5) / 6, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, kOps, 0);
+    if constexpr (!kAhead) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    if constexpr (!kAhead) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
   }
 }
 
-// Whether any lane's accumulators hold what the split cannot vouch for: a
-// non-finite value, or a nonzero one below 2^-100. Uniform per wavefront.
-__device__ __forceinline__ bool AnySuspect(const floatx16& acc) {
-  uint32_t low = ~0u;  // min over (|c| bits << 1) - 1; zero wraps to the top
-  float nonfinite = 0.0f;
+// Whether any lane's accumulators hold a non-finite value. Uniform per
+// wavefront.
+__device__ __forceinline__ bool AnyNonFinite(const floatx16& acc) {
+  float x = 0.0f;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const float c = acc[v];
-    low = std::min(low, (__builtin_bit_cast(uint32_t, c) << 1) - 1u);
-    nonfinite = __builtin_fmaf(c, 0.0f, nonfinite);
-  }
-  constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1u;
-  return __ballot(low < kTiny || !(nonfinite == 0.0f)) != 0;
+  for (int v = 0; v < 16; ++v) x = __builtin_fmaf(acc[v], 0.0f, x);
+  return __ballot(!(x == 0.0f)) != 0;
 }
 
 struct GemmKArgs {
@@ -382,7 +392,12 @@ struct Stage {
 
   // Vector i, `back` bytes before its place.
   __device__ __forceinline__ void load_vec(int i, GlobalPtr<T> org, Off back = 0) {
-    const GlobalPtr<char> src = (GlobalPtr<char>)org + (off[i] - back);
+    Off o = off[i] - back;
+    // Bound to the stage's origin here: with the 32-bit offset's extension
+    // hoisted out of the loop, every load took a 64-bit vector addition and
+    // two offset registers (8-36 bytes of scratch on the largest tiles).
+    if constexpr (VEC) asm("" : "+v"(o) : "s"(org));
+    const GlobalPtr<char> src = (GlobalPtr<char>)org + o;
     if constexpr (kF32) {
       using V = typename std::conditional<VEC, floatx4, floatx4u>::type;
       const V q = *(GlobalPtr<V>)src;
@@ -502,8 +517,13 @@ struct Stage {
         for (int e = 0; e < 4; ++e) q[e] = static_cast<float>(static_cast<int8_t>(w >> (8 * e)));
       }
       uint32_t lo[3], hi[3];
-      Split2(q[0], q[1], lo);
-      Split2(q[2], q[3], hi);
+      if constexpr (kF32) {
+        Split2(q[0], q[1], lo);
+        Split2(q[2], q[3], hi);
+      } else {
+        lo[0] = Exact2(q[0], q[1]);
+        hi[0] = Exact2(q[2], q[3]);
+      }
 #pragma unroll
       for (int part = 0; part < kParts; ++part)
         *reinterpret_cast<uint2*>(dst + part * kPlane) = make_uint2(lo[part], hi[part]);
@@ -673,21 +693,39 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     xa.load_full(ScalarBase(a_org + s * a_step));
     xb.load_full(ScalarBase(b_org + s * b_step));
   };
+  // kOneSet (the tiles of 64x64 wavefronts): their accumulators leave registers
+  // for one stage set only. Each vector of stage t + 1 is split and stored
+  // between the MFMAs of stage t, and its registers take stage t + 2's load at
+  // once.
+  constexpr bool kOneSet = BM * BN >= 4;
+  // Interleave's room for the split. Beyond its 26 operations, more lets the
+  // split run ahead of its share, which pays where fragments are read with one
+  // LDS read each and on the 64x64-wavefront tiles; the transposing reads'
+  // tiles wait longer for their first fragments with it (us at 24 | 40, at
+  // 8192x2048x2048: NT 128x64 428 | 402, 256x128 362 | 335; NN 128x128 of four
+  // wavefronts 432 | 404, 256x128 362 | 348; TN 256x128 344 | 363; 128x64 NN
+  // 530 | 545, TN 532 | 562).
+  constexpr int kSplitOps = BM * BN == 1 ? 28
+                            : (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
+                                                                           : 24;
   // Steady-state iteration on stage t (t + 2 < nfull): load stage t + 2 into
   // set `ld`, contract stage t, store stage t + 1 from set `st`. With VEC the
   // body is one basic block, scheduled as one interleave.
   auto steady = [&](StageA& lda_, StageB& ldb_, const StageA& sta, const StageB& stb,
                     int64_t t, int cur, auto fold) {
     load_full(lda_, ldb_, t + 2);
+    // One block per wavefront: the loads go out first. Placed by the scheduler
+    // they went out late in the stage, and the next one began by waiting for
+    // them (us, as scheduled | loads first, NN, NT, TN: 1024x1024x2048 49, 44,
+    // 50 | 38, 38, 42; 64x64x512 12.5, 12.8, 12.3 | 11.5, 11.4, 12.5;
+    // 2048x1376x512 30.6, 27.8, 31.5 | 29.6, 27.8, 30.9).
+    constexpr bool kAhead = BM * BN == 1;
+    if constexpr (kAhead) __builtin_amdgcn_sched_barrier(0);
     compute(a_buf(cur), b_buf(cur), fold);
     sta.store(a_buf(cur ^ 1));
     stb.store(b_buf(cur ^ 1));
-    // One block per wavefront leaves too few MFMAs to hide the split under:
-    // there the scheduler's own order is the faster (64x64 tiles on
-    // 2048x512x1376: 27 us, interleaved 29; 128x64 tiles: 37, interleaved 33).
-    if constexpr (BM * BN > 1)
-      Interleave<(KT / KG) * BM * BN*(PB == 3 ? 6 : 3), StageA::kPer + StageB::kPer,
-                 BM * 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2)>();
+    Interleave<(KT / KG) * BM * BN*(PB == 3 ? 6 : 3), StageA::kPer + StageB::kPer,
+               BM * 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2), kSplitOps, kAhead>();
     __syncthreads();
   };
 
@@ -714,11 +752,6 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       t[e] = in ? x : 0.0f;
     }
   };
-  // kOneSet (the tiles of 64x64 wavefronts): their accumulators leave registers
-  // for one stage set only. Each vector of stage t + 1 is split and stored
-  // between the MFMAs of stage t, and its registers take stage t + 2's load at
-  // once.
-  constexpr bool kOneSet = BM * BN >= 4;
   int64_t t = 0;
   if constexpr (kOneSet) {
     constexpr int kVA = StageA::kPer, kV = kVA + StageB::kPer;
@@ -755,7 +788,8 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
             }
           }
         }
-        Interleave<BM * BN*(PB == 3 ? 6 : 3), kV, 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2)>();
+        Interleave<BM * BN*(PB == 3 ? 6 : 3), kV, 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2), kSplitOps,
+                   false>();
         __syncthreads();
       };
       for (; t + kPerChunk + 1 < nfull; t += kPerChunk) {  // a chunk
@@ -823,16 +857,17 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
 #pragma unroll
     for (int j = 0; j < BN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v] + acc[i][j][v];
+      for (int v = 0; v < 16; ++v)
+        acc[i][j][v] = (B_I8 ? kOpUnscale : kOpUnscale * kOpUnscale) * (sum[i][j][v] + acc[i][j][v]);
 
-  // Recompute: a suspect block's outputs by fp32 products, straight from
+  // Recompute: a non-finite block's outputs by fp32 products, straight from
   // memory (k pairs 16g + j, 16g + 8 + j). Decided per 32x32 block of the
   // output, so that it does not depend on the tile config.
 #pragma unroll
   for (int i = 0; i < BM; ++i)
 #pragma unroll
     for (int j = 0; j < BN; ++j)
-      if (__builtin_expect(AnySuspect(acc[i][j]), false)) {
+      if (__builtin_expect(AnyNonFinite(acc[i][j]), false)) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
         const int64_t m = std::min<int64_t>(m0 + wm0 + 32 * i + r, p.M - 1);
@@ -881,7 +916,9 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
         floatx16 ua[1][1] = {}, before[1][1] = {};
         MfmaStep<true>(fa, fb, ua, before);
         floatx16& u = ua[0][0];
-        if (__builtin_expect(AnySuspect(u), false)) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) u[v] *= kOpUnscale * kOpUnscale;
+        if (__builtin_expect(AnyNonFinite(u), false)) {
 #pragma unroll
           for (int v = 0; v < 16; ++v) u[v] = 0.0f;
 #pragma unroll

@@ -125,3 +125,74 @@ def test_values_the_split_cannot_hold(gpu, kind):
                               clean.cpu().numpy().reshape(M, N)[keep].view(np.uint32)), cfg
         first = got if first is None else first
         assert np.array_equal(got.view(np.uint32), first.view(np.uint32)) or kind == "nan", cfg
+
+
+# Exponents of A's and B's values: A under bf16's smallest parts (2^-133) and
+# subnormal, lifted by B; both small, with subnormal results; and operands and
+# results past the scaled split's range (2^103, 2^80), which are recomputed.
+RANGES = [(-112, 20), (-120, 24), (-126, 40), (-136, 60), (-146, 100), (30, -130), (-70, -70),
+          (90, 20), (108, -30)]
+
+
+def in_range(got, want, K, roundings=1):
+    """The split's bound, or the fp32 MFMA's on recomputed blocks (K rounded
+    terms), and `roundings` of fp32's smallest subnormal."""
+    err = np.linalg.norm(got.astype(np.float64) - want)
+    return err <= np.sqrt(96 + K) * 2.0 ** -24 * np.linalg.norm(want) + roundings * np.sqrt(want.size) * 2.0 ** -149
+
+
+@pytest.mark.parametrize("ea,eb", RANGES)
+def test_operands_of_every_magnitude(gpu, ea, eb):
+    """Operands keep all 24 bits at every magnitude (subnormals those they
+    have) whatever the other operand's, on every tile config, layout and load
+    form, with split-K, int8 weights, scaled loads and in the LoRA epilogue."""
+    torch, L = gpu
+    r = np.random.default_rng([ea + 200, eb + 200])
+    draw = lambda e, *shape: np.ldexp(r.standard_normal(shape), e).astype(f32)  # noqa: E731
+    wide = lambda x: x.astype(np.float64)  # noqa: E731
+    empty = lambda n: torch.full((n,), 7.0, device="cuda:0")  # noqa: E731
+    M, N, K = 200, 136, 328
+    A, B = draw(ea, M, K), draw(eb, K, N)
+    want = wide(A) @ wide(B)
+    for layout in range(3):
+        a = device(torch, np.ascontiguousarray(A.T if layout == 2 else A).ravel(), 0)
+        b = device(torch, np.ascontiguousarray(B.T if layout == 1 else B).ravel(), 0)
+        for cfg in range(L.seeml_hip_gemm_config_count() - 1):
+            for splits in (1, 3):
+                out = empty(M * N)
+                call(gpu, "gemm_forced", layout, a, b, out, M, N, K, cfg, splits)
+                assert in_range(out.cpu().numpy().reshape(M, N), want, K, splits), (layout, cfg, splits)
+    # the general form's two tiles
+    for cfg in (0, 5):
+        M, N, K = 131, 67, 77
+        A, B = draw(ea, M, K), draw(eb, K, N)
+        want = wide(A) @ wide(B)
+        for layout in range(3):
+            a = device(torch, np.ascontiguousarray(A.T if layout == 2 else A).ravel(), 1)
+            b = device(torch, np.ascontiguousarray(B.T if layout == 1 else B).ravel(), 1)
+            out = empty(M * N)
+            call(gpu, "gemm_forced", layout, a, b, out, M, N, K, cfg, 1)
+            assert in_range(out.cpu().numpy().reshape(M, N), want, K), (layout, cfg)
+    # int8 weights under a scale of B's exponent
+    Q, scale = r.integers(-128, 128, (K, N)).astype(np.int8), f32(np.ldexp(1.0, max(eb - 7, -120)))
+    out = empty(M * N)
+    call(gpu, "gemm_nn_q8", device(torch, A.ravel(), 0), device(torch, Q.ravel(), 0), out, M, N, K,
+         float(scale), 0)
+    assert in_range(out.cpu().numpy().reshape(M, N), float(scale) * (wide(A) @ wide(Q)), K, 1 + scale)
+    # scaled loads: the factor brings the stream to A's exponent
+    M, N, K, s = 256, 64, 328, f32(np.ldexp(0.75, max(ea, -140) // 2))
+    A, B = draw(max(ea, -140) - max(ea, -140) // 2, M, K), draw(eb, N, K)
+    for cfg in (4, 5, 8, 9, 10, 11):
+        out = empty(M * N)
+        call(gpu, "gemm_forced_scaled", 1, device(torch, A.ravel(), 0), device(torch, B.ravel(), 0), out,
+             M, N, K, cfg, 1, float(s))
+        assert in_range(out.cpu().numpy().reshape(M, N), wide(s * A) @ wide(B).T, K), cfg
+    # the LoRA epilogue over a zero base product
+    M, N, K, rank = 300, 264, 64, 16
+    T, Bl = draw(ea, M, rank), draw(eb, rank, N)
+    zero, w = device(torch, np.zeros(M * K, f32), 0), device(torch, draw(0, N, K).ravel(), 0)
+    for cfg in (0, 2, 4, 5, 8, 9):
+        out = empty(M * N)
+        call(gpu, "gemm_forced_lora", 1, zero, w, out, M, N, K, cfg, 0, 0, device(torch, T.ravel(), 0),
+             device(torch, Bl.ravel(), 0), rank, 0, 1.0, 1)
+        assert in_range(out.cpu().numpy().reshape(M, N), wide(T) @ wide(Bl), rank), cfg
