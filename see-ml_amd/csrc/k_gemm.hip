@@ -78,22 +78,53 @@ namespace {
 // The tile of a GEMM by how many workgroups each leaves for the chip's 256
 // CUs. A larger tile reads its operands less often and splits them less per
 // product, and loses more to a last round of the chip that it leaves partly
-// idle. Measured on NT, one slice (us; 256x128 | 128x128 | 128x64 | 64x64):
-//   8192x2048x2048 339 | 358 | 430 | 452    2048x2048x2048 132 | 103 | 116 | 124
-//   2048x5504x2048 296 | 269 | 309 | 319    2048x1376x512   45 |  36 |  30 |  27
-//   2048x512x1376   87 |  63 |  44 |  31    600x4096x1024   75 |  60 |  53 |  45
-// So: 256x128 from rounds filled to 7/8 on, 128x128 from nearly a workgroup per
-// CU on, else 64x64 (the 128x64 tiles only where 64x64 would pass two per CU).
-int TileFor(const GemmDesc& d) {
-  if (d.N <= 32 && d.M > 32) return gemm::kCfgSkinnyN;
-  if (d.M <= 32 && d.N > 32) return gemm::kCfgSkinnyM;
-  auto tiles = [&](int64_t m, int64_t n) { return CeilDiv(d.M, m) * CeilDiv(d.N, n) * d.batch; };
+// idle, to the part of a tile beyond the output, and to the general write-back
+// of partial tiles (5-6 us). Measured, one slice, us, NN:
+//                 256x128 128x128 64x64 64x64x16              256x128 128x128 64x64 64x64x16
+//   8192x2048x2048  355     404    --     --    2048x2752x64    18.9   20.4   15.5   13.7
+//   2560x2560x512    44      48    57     56    744x5496x400    41.4   43.7   41.3   37.4
+//   2048x2048x2048  139     110   122    122    2048x2752x512   48.2   52.7   48.9   48.2
+//   2048x2752x2048  146     162   172    171    2948x1216x236   30.2   26.6   23.0   19.4
+//   1024x1024x2048  137     102    42     48    744x5496x2048    145    153    146    144
+//   60000x64x256     35      37    26     24    64x65536x512     105     60     38     41
+// So: 256x128 from rounds filled to 7/8 on. 128x128 from nearly a workgroup per
+// CU on, except below 7/8 of two per CU with partial tiles on a short reduction
+// or just past a round. Else 64x64 (128x64 where 64x64 would pass two per CU).
+// Outputs up to 64 wide or tall take 64x64. So do causal attention products,
+// which skip per tile, below two 128x128 tiles per CU, unless they are tall and
+// fill those tiles (one tile per CU, us, 128x128 | 64x64: 16x128x16x80 dQ 24 | 18,
+// 2x2000x8x80 dQ 113 | 93; 2x1023x16x128 dQ 58 | 66).
+// The 64x64 tile is 16 deep where a reduction of at most 128 has more of them
+// than the three per CU that the LDS of the 32-deep one allows (3008x1984x64
+// above; the deeper one has the LoRA and group kernels too), and 128x128 of
+// eight wavefronts where short split-K slices make that many of filled ones
+// (512x512x2048 in 16 slices 32 -> 26 us; 654x1177x6120 in 5 101 -> 122).
+// Outputs up to 32 take the 32-wide tiles except with split-K at a workgroup
+// per CU at most, where the 64x64 tile's stages are shorter (32x256x512 in two
+// slices 12.0 -> 11.0 us; unsplit, its partial tiles pay the general write-back).
+int TileFor(const GemmDesc& d, int splits) {
   constexpr int64_t kCus = 256, kMost = kCus * 7 / 8;
-  const int64_t large = tiles(256, 128);
-  if (d.causal == Causal::kNone && large * 8 >= CeilDiv(large, kCus) * kCus * 7) return gemm::kCfgLarge;
-  if (tiles(128, 128) >= kMost) return gemm::kCfgDefault;
+  auto tiles = [&](int64_t m, int64_t n) { return CeilDiv(d.M, m) * CeilDiv(d.N, n) * d.batch; };
+  const int64_t small_groups = tiles(64, 64) * splits;
+  if ((d.N <= 32) != (d.M <= 32) && !(splits > 1 && small_groups <= kCus))
+    return d.N <= 32 ? gemm::kCfgSkinnyN : gemm::kCfgSkinnyM;
+  const bool narrow = d.M <= 64 || d.N <= 64;
+  const bool fills = CeilDiv(d.N, 128) * 128 * 7 <= d.N * 8 && CeilDiv(d.M, 128) * 128 * 7 <= d.M * 8;
+  if (splits > 1 && fills && small_groups > 3 * kCus && d.K <= 256 * int64_t{splits}) return gemm::kCfgWaves8;
+  const int small = d.K <= 128 && small_groups > 3 * kCus ? gemm::kCfgSmallK16 : gemm::kCfgSmall;
+  if (narrow) return small;
+  const int64_t large = tiles(256, 128), mid = tiles(128, 128);
+  if (d.causal != Causal::kNone) {
+    return mid >= 2 * kCus || (mid >= kMost && fills && d.M >= 4 * 128) ? gemm::kCfgDefault : small;
+  }
+  if (large * 8 >= CeilDiv(large, kCus) * kCus * 7) return gemm::kCfgLarge;
+  if (mid >= kMost) {
+    const bool partial = d.M % 128 != 0 || d.N % 128 != 0;
+    const bool just_past = mid > kCus && mid < kCus * 5 / 4;
+    return partial && mid < 2 * kMost && (d.K <= 512 || just_past) ? small : gemm::kCfgDefault;
+  }
   if (tiles(128, 64) >= 2 * kMost) return gemm::kCfgHalf;
-  return gemm::kCfgSmall;
+  return small;
 }
 
 // Split-K slices, part of a shape's summation order. The rank-wide outputs of
@@ -138,11 +169,11 @@ GemmPlan PlanGemmWith(const GemmDesc& d, int forced_cfg, int forced_splits) {
     plan.ws_bytes = SkinnyWorkspace(d);
     return plan;
   }
-  plan.cfg = forced_cfg >= 0 && forced_cfg < kNumCfgs ? forced_cfg : TileFor(d);
   if (forced_splits >= 1)
     plan.splits = d.batch == 1 && d.causal == Causal::kNone ? forced_splits : 1;
   else
     plan.splits = SplitsFor(d, kind);
+  plan.cfg = forced_cfg >= 0 && forced_cfg < kNumCfgs ? forced_cfg : TileFor(d, plan.splits);
   plan.ws_bytes = plan.splits > 1 ? static_cast<size_t>(plan.splits) * d.M * d.N * sizeof(float) : 0;
   return plan;
 }

@@ -313,7 +313,7 @@ inline constexpr CfgInfo kCfgs[] = {
 constexpr int MinWaves(int mt_m, int mt_n) { return mt_m * mt_n >= 128 * 128 ? 2 : 1; }
 inline constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
 inline constexpr int kCfgDefault = 0, kCfgSmall = 5, kCfgSkinnyN = 6, kCfgSkinnyM = 7,
-                     kCfgLarge = 2, kCfgHalf = 9;
+                     kCfgLarge = 2, kCfgWaves8 = 1, kCfgHalf = 9, kCfgSmallK16 = 10;
 
 // One operand's MT x KT stage (outer index o = m for A / n for B), held in
 // registers between its global loads and its LDS store, where it is split.
@@ -725,7 +725,7 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   // wavefronts 432 | 404, 256x128 362 | 348; TN 256x128 344 | 363; 128x64 NN
   // 530 | 545, TN 532 | 562).
   constexpr int kSplitOps = BM * BN == 1 ? 28
-                            : (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
+                            : VEC && (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
                                                                            : 24;
   // Steady-state iteration on stage t (t + 2 < nfull): load stage t + 2 into
   // set `ld`, contract stage t, store stage t + 1 from set `st`. With VEC the
@@ -738,13 +738,15 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     // them (us, as scheduled | loads first, NN, NT, TN: 1024x1024x2048 49, 44,
     // 50 | 38, 38, 42; 64x64x512 12.5, 12.8, 12.3 | 11.5, 11.4, 12.5;
     // 2048x1376x512 30.6, 27.8, 31.5 | 29.6, 27.8, 30.9).
-    constexpr bool kAhead = BM * BN == 1;
+    // (1000x770x1531 layer 116 -> 111.) An int8 operand leaves too few MFMAs.
+    constexpr bool kAhead = BM * BN == 1 && PB == 3;
     if constexpr (kAhead) __builtin_amdgcn_sched_barrier(0);
     compute(a_buf(cur), b_buf(cur), fold);
     sta.store(a_buf(cur ^ 1));
     stb.store(b_buf(cur ^ 1));
-    Interleave<(KT / KG) * BM * BN*(PB == 3 ? 6 : 3), StageA::kPer + StageB::kPer,
-               BM * 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2), kSplitOps, kAhead>();
+    if constexpr (kAhead || BM * BN > 1)
+      Interleave<(KT / KG) * BM * BN*(PB == 3 ? 6 : 3), StageA::kPer + StageB::kPer,
+                 BM * 3 * (A_KC ? 1 : 2) + BN * PB * (B_KC ? 1 : 2), kSplitOps, kAhead>();
     __syncthreads();
   };
 

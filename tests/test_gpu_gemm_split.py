@@ -8,6 +8,8 @@ rounded terms per 16 k within a chunk of 64, then one per chunk; each rounding
 is at most 2^-24 of a partial sum, so the relative 2-norm error of a random
 product stays below sqrt(24 * 4 + K / 64) * 2^-24 (6e-7 at K = 64, 8e-7 at
 K = 4096)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -196,3 +198,17 @@ def test_operands_of_every_magnitude(gpu, ea, eb):
         call(gpu, "gemm_forced_lora", 1, zero, w, out, M, N, K, cfg, 0, 0, device(torch, T.ravel(), 0),
              device(torch, Bl.ravel(), 0), rank, 0, 1.0, 1)
         assert in_range(out.cpu().numpy().reshape(M, N), wide(T) @ wide(Bl), rank), cfg
+
+
+def test_narrow_outputs_take_narrow_tiles(gpu):
+    """Every GEMM of this plan has an output at most 64 wide over 60000 rows:
+    no tile may be wider than 64 both ways, however many of them there are."""
+    from seeml_amd import DeviceUpdateEngine, PROGRAM_TRAIN, configs, planner
+    cfg = planner.UpdateConfig(batch=60000, loss="xent", lr=1e-3,
+                               lora=planner.LoraSpec(rank=8, alpha=16.0, seed=7))
+    plan = planner.compile_update(configs.mlp_model(64, 64, 48), cfg)
+    e = DeviceUpdateEngine(plan.blob)
+    e.build()
+    tiles = [re.search(r"(\d+)x(\d+)x\d+/", e.gemm_choice(PROGRAM_TRAIN, i)) for i in range(len(plan.train))]
+    tiles = [(int(t[1]), int(t[2])) for t in tiles if t]
+    assert tiles and all(min(t) <= 64 for t in tiles), tiles
