@@ -132,26 +132,22 @@ int TileFor(const GemmDesc& d, int splits) {
 // long reduction, and so have outputs of at most 64 tiles: enough slices to
 // cover the chip twice with 64x64 or 128x128 tiles, each at least 128 deep.
 // Elsewhere a slice costs a pass over the output and a launch (about 5 us),
-// against about 0.6 us per 32 of depth that a lone workgroup takes: slices of
-// 1024, no more than two 128x128 tiles' worth per CU, where the output leaves
-// CUs idle (600x1024x1024 takes 24 us in one slice, 600x1024x4096 82 us in one
-// and 48 in four), otherwise none.
+// against about 0.55 us per 32 of depth that a lone workgroup takes: slices of
+// 1024, no more than two 128x128 tiles' worth per CU (64x64 tiles' for outputs
+// up to 64 wide or tall), where the output leaves CUs idle (600x1024x1024 takes
+// 23 us in one slice, 600x1024x4096 82 us in one and 48 in four), otherwise none.
+// No shape takes more slices than 128-deep ones covering the chip twice.
 int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
   if (d.batch != 1 || d.causal != Causal::kNone || d.K < 256) return 1;
   const int64_t big = CeilDiv(d.M, 128) * CeilDiv(d.N, 128), mid = CeilDiv(d.M, 64) * CeilDiv(d.N, 64);
-  int64_t tiles = mid;
-  if (kind == SkinnyKind::kRowDot || kind == SkinnyKind::kColSum || mid <= 64) {
-    tiles = d.N <= 32 && d.M > 32   ? CeilDiv(d.M, 128)
-            : d.M <= 32 && d.N > 32 ? CeilDiv(d.N, 128)
-            : big >= 512 || (mid < 256 && d.M > 64 && d.N > 64) ? big : mid;
-  } else if (mid < 256) {
-    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(d.K / 1024, CeilDiv(512, big))));
-  } else {
-    return 1;
-  }
+  const bool narrow = d.M <= 64 || d.N <= 64;
+  const int64_t tiles = d.N <= 32 && d.M > 32   ? CeilDiv(d.M, 128)
+                        : d.M <= 32 && d.N > 32 ? CeilDiv(d.N, 128)
+                        : big >= 512 || (mid < 256 && !narrow) ? big : mid;
   if (tiles >= 512) return 1;
-  const int64_t want = CeilDiv(512, tiles), most = d.K / 128;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(most, 64))));
+  int64_t most = d.K / 128;
+  if (kind != SkinnyKind::kRowDot && kind != SkinnyKind::kColSum && mid > 64) most = mid < 256 ? d.K / 1024 : 1;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(CeilDiv(512, tiles), std::min<int64_t>(most, 64))));
 }
 }  // namespace
 

@@ -212,3 +212,26 @@ def test_narrow_outputs_take_narrow_tiles(gpu):
     tiles = [re.search(r"(\d+)x(\d+)x\d+/", e.gemm_choice(PROGRAM_TRAIN, i)) for i in range(len(plan.train))]
     tiles = [(int(t[1]), int(t[2])) for t in tiles if t]
     assert tiles and all(min(t) <= 64 for t in tiles), tiles
+
+
+@pytest.mark.parametrize("wide", [33, 48, 64])
+def test_split_k_scratch_stays_within_the_covering_slices(gpu, wide):
+    """A shape takes no more scratch than 128-deep slices covering the chip
+    twice would: gemm_tn_noalloc serves every shape whose need by that count
+    fits its array, with gemm_tn's bits."""
+    from test_gpu_kernels import heuristic_splits
+    torch, _ = gpu
+    g = torch.Generator(device="cuda:0").manual_seed(wide)
+    a, b = (torch.randn(8192 * 16400, device="cuda:0", generator=g) for _ in range(2))
+    served = 0
+    for other in (4097, 4801, 8193, 12290, 16399):
+        for K in (1030, 4096, 8192):
+            for M, N in ((wide, other), (other, wide)):
+                if heuristic_splits(M, N, K) * M * N * 4 > 16 << 20:
+                    continue
+                want, got = (torch.empty(M * N, device="cuda:0") for _ in range(2))
+                call(gpu, "gemm_tn", a, b, want, M, N, K)
+                call(gpu, "gemm_tn_noalloc", a, b, got, M, N, K)
+                assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (M, N, K)
+                served += 1
+    assert served >= 6
