@@ -135,8 +135,10 @@ int TileFor(const GemmDesc& d, int splits) {
 // against about 0.55 us per 32 of depth that a lone workgroup takes: slices of
 // 1024, no more than two 128x128 tiles' worth per CU (64x64 tiles' for outputs
 // up to 64 wide or tall), where the output leaves CUs idle (600x1024x1024 takes
-// 23 us in one slice, 600x1024x4096 82 us in one and 48 in four), otherwise none.
-// No shape takes more slices than 128-deep ones covering the chip twice.
+// 23 us in one slice, 600x1024x4096 82 us in one and 48 in four); two of at least 2048 up to
+// two 64x64 tiles per CU (in one and two slices, us, NN: 1024x1024x8192 137 and
+// 126, x4096 74 and 70, x2048 39 and 40; 1280x1024x8192 202 and 180); otherwise
+// none. No shape takes more slices than 128-deep ones covering the chip twice.
 int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
   if (d.batch != 1 || d.causal != Causal::kNone || d.K < 256) return 1;
   const int64_t big = CeilDiv(d.M, 128) * CeilDiv(d.N, 128), mid = CeilDiv(d.M, 64) * CeilDiv(d.N, 64);
@@ -146,7 +148,7 @@ int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
                         : big >= 512 || (mid < 256 && !narrow) ? big : mid;
   if (tiles >= 512) return 1;
   int64_t most = d.K / 128;
-  if (kind != SkinnyKind::kRowDot && kind != SkinnyKind::kColSum && mid > 64) most = mid < 256 ? d.K / 1024 : 1;
+  if (kind != SkinnyKind::kRowDot && kind != SkinnyKind::kColSum && mid > 64) most = mid < 256 ? d.K / 1024 : d.K / 2048;
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(CeilDiv(512, tiles), std::min<int64_t>(most, 64))));
 }
 }  // namespace
