@@ -34,10 +34,10 @@
 // three smallest are at most 2^-26 of the whole, a quarter of the fp32
 // product's own rounding, and are left out; the other six run as six
 // v_mfma_f32_32x32x16_bf16 into one fp32 accumulator, smallest first. The
-// accumulator is added to a second one and cleared every 64 k (kChunk): the
-// bf16 MFMA's own additions lean slightly to one side, which a sum over many
-// rows of such results would show, and short sums keep that and the rounding
-// small. Relative 2-norm error against 64 bits, fp32 MFMA | this: normal
+// accumulator is added to a second one and cleared every 64 k (kChunk), which
+// keeps the rounding small. The bf16 MFMA's own additions lean to one side;
+// half of the rows are computed negated, so that a sum over many rows of such
+// results does not add the lean up (RowNegated below). Relative 2-norm error against 64 bits, fp32 MFMA | this: normal
 // operands K = 16 7.4e-8 | 3.3e-8, K = 2048 8.1e-7 | 1.6e-7, K = 8192 1.62e-6 |
 // 2.5e-7; softmax gradients times a head of 8192 classes 1.6e-6 | 2.3e-7;
 // log-normal operands 6.6e-7 | 1.3e-7 (without the second accumulator 7.0e-7
@@ -140,9 +140,10 @@ __device__ __forceinline__ GlobalPtr<T> ScalarBase(const T* p) {
 constexpr float kOpScale = 0x1p24f;
 template <int PB>  // parts of B
 constexpr float kUnscale = PB == 3 ? 0x1p-48f : 0x1p-24f;
-__device__ __forceinline__ void Split2(float x0, float x1, uint32_t (&p)[3]) {
-  x0 *= kOpScale;
-  x1 *= kOpScale;
+__device__ __forceinline__ void Split2(float x0, float x1, uint32_t (&p)[3], float s0 = kOpScale,
+                                       float s1 = kOpScale) {
+  x0 *= s0;
+  x1 *= s1;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const bf16x2 h = __builtin_convertvector((floatx2){x0, x1}, bf16x2);
@@ -160,13 +161,22 @@ __device__ __forceinline__ uint32_t Exact2(float x0, float x1) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x0, x1}, bf16x2));
 }
 
+// Half of A's rows are negated on the way in, and their sums on the way out:
+// the bf16 MFMA rounds towards minus infinity, a lean of up to 6e-8 of the
+// outputs' size that a sum over many rows (a weight gradient's) would add up
+// and that the two signs cancel. Which half costs no vector register in each
+// layout: k-contiguous, every other 64 rows, one sign per wavefront on the way
+// out and per vector on the way in; row-contiguous, the odd rows, one sign per
+// element.
+constexpr bool RowNegated(int64_t m) { return (m >> 6) & 1; }
+
 // The parts of a lane's 8 consecutive k.
-__device__ __forceinline__ void Split8(const float* x, bf16x8 (&f)[3]) {
+__device__ __forceinline__ void Split8(const float* x, bf16x8 (&f)[3], float scale) {
   uint32_t w[3][4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     uint32_t p[3];
-    Split2(x[2 * q], x[2 * q + 1], p);
+    Split2(x[2 * q], x[2 * q + 1], p, scale, scale);
 #pragma unroll
     for (int part = 0; part < 3; ++part) w[part][q] = p[part];
   }
@@ -179,11 +189,11 @@ __device__ __forceinline__ void Split8(const float* x, bf16x8 (&f)[3]) {
 // products of NA = NB = 3 parts, or the three of an exact (one-part) B,
 // smallest first, each over all blocks so that consecutive MFMAs are
 // independent. FOLD: the first step of a chunk (kChunk): the accumulators,
-// holding the chunk before, are added to `sum`, unscaled, and start again
-// from zero.
-template <bool FOLD, int BM, int BN, int PB>
+// holding the chunk before, are added to `sum`, unscaled (with the rows'
+// sign), and start again from zero.
+template <bool FOLD, bool A_KC, int BM, int BN, int PB>
 __device__ __forceinline__ void MfmaStep(const bf16x8 (&fa)[BM][3], const bf16x8 (&fb)[BN][PB],
-                                         floatx16 (&acc)[BM][BN], floatx16 (&sum)[BM][BN]) {
+                                         floatx16 (&acc)[BM][BN], floatx16 (&sum)[BM][BN], float unscale) {
   constexpr int kProducts = PB == 3 ? 6 : 3;
   constexpr int ia[6] = {2, PB == 3 ? 0 : 1, PB == 3 ? 1 : 0, 1, 0, 0};
   constexpr int ib[6] = {0, PB == 3 ? 2 : 0, PB == 3 ? 1 : 0, 0, PB == 3 ? 1 : 0, 0};
@@ -197,7 +207,7 @@ __device__ __forceinline__ void MfmaStep(const bf16x8 (&fa)[BM][3], const bf16x8
         if (FOLD && q == 0) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            sum[i][j][v] = __builtin_fmaf(acc[i][j][v], kUnscale<PB>, sum[i][j][v]);
+            sum[i][j][v] = __builtin_fmaf(acc[i][j][v], !A_KC && v & 1 ? -unscale : unscale, sum[i][j][v]);
         }
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             fa[i][ia[q]], fb[j][ib[q]], FOLD && q == 0 ? kZero : acc[i][j], 0, 0, 0);
@@ -336,7 +346,7 @@ inline constexpr int kCfgDefault = 0, kCfgSmall = 5, kCfgSkinnyN = 6, kCfgSkinny
 // waited for anyway (scaled as loaded, each stage's loads would be waited
 // for at once, a stage early: 2.5x slower on the rank-64 shapes); a final
 // partial stage is scaled as loaded, under its in-range masks.
-template <int MT, int KT, bool KC, typename T, int NT, bool VEC, bool SC = false>
+template <int MT, int KT, bool KC, typename T, int NT, bool VEC, bool IS_A, bool SC = false>
 struct Stage {
   static constexpr bool kF32 = std::is_same<T, float>::value;
   static constexpr int kParts = kF32 ? 3 : 1;
@@ -346,6 +356,12 @@ struct Stage {
   static constexpr int kPer = kVecs / NT;
   static_assert(kVecs % NT == 0, "stage shape");
   static_assert(!SC || VEC, "scaled loads need the vector form");
+  // k-contiguous: rows between a thread's vectors (its first is below 64, or
+  // below 128 with the step of 128), so that a vector's rows share a sign, and
+  // whether the first one's sign depends on the tile or the wavefront.
+  static constexpr int kRowStep = NT / (KT / 4);
+  static constexpr bool kRowBase = IS_A && KC && (MT < 128 || kRowStep == 128);
+  static_assert(!IS_A || !KC || kRowStep == 32 || kRowStep == 64 || kRowStep == 128, "one sign per vector");
   static_assert(!VEC || kF32, "int8 operands take the general form");
   float r[kPer][4];
   // Byte offset of vector i from the stage origin. VEC: the host checks that
@@ -356,6 +372,7 @@ struct Stage {
   int shift[kPer];    // !VEC, row-contiguous: places the vector was read back by
   int avail;          // !VEC, row-contiguous: elements of the row from the tile's start on
   bool few;           // !VEC, row-contiguous: rows of fewer than 4 elements
+  uint32_t rs;        // kRowBase: the scale with the first vector's rows' sign, as bits
   float sc;           // SC: the factor
   bool pend;          // SC: loaded unscaled (a whole stage), scaled at the store
 
@@ -371,6 +388,10 @@ struct Stage {
 
   // o0: first row of the tile (a multiple of 4); oe: the operand's extent.
   __device__ __forceinline__ void init(int64_t ld, int64_t o0, int64_t oe) {
+    if constexpr (kRowBase) {
+      const int first = kRowStep == 128 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) * 64 : 0;
+      rs = __builtin_bit_cast(uint32_t, kOpScale) | static_cast<uint32_t>(RowNegated(o0 + first)) << 31;
+    }
     // >= 1: the tile starts in range.
     const int left = static_cast<int>(std::min<int64_t>(oe - o0, MT));
     if constexpr (!VEC && !KC) {
@@ -516,8 +537,17 @@ struct Stage {
       }
       uint32_t lo[3], hi[3];
       if constexpr (kF32) {
-        Split2(q[0], q[1], lo);
-        Split2(q[2], q[3], hi);
+        float s0 = kOpScale, s1 = IS_A && !KC ? -kOpScale : kOpScale;
+        if constexpr (IS_A && KC) {
+          if constexpr (kRowBase) {
+            uint32_t bits = rs;
+            asm("" : "+s"(bits));  // kept in a scalar register
+            s0 = __builtin_bit_cast(float, bits);
+          }
+          s0 = s1 = RowNegated(i * kRowStep) ? -s0 : s0;
+        }
+        Split2(q[0], q[1], lo, s0, s1);
+        Split2(q[2], q[3], hi, s0, s1);
       } else {
         lo[0] = Exact2(q[0], q[1]);
         hi[0] = Exact2(q[2], q[3]);
@@ -591,8 +621,8 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   static_assert(WM % 32 == 0 && WN % 32 == 0 && KT % KG == 0 && kSplitAlign % KT == 0,
                 "tile shape");
   constexpr bool kVecB = VEC && !B_I8;
-  using StageA = Stage<MT_M, KT, A_KC, float, NT, VEC, SCL == 1>;
-  using StageB = Stage<MT_N, KT, B_KC, BT, NT, kVecB, SCL == 2>;
+  using StageA = Stage<MT_M, KT, A_KC, float, NT, VEC, true, SCL == 1>;
+  using StageB = Stage<MT_N, KT, B_KC, BT, NT, kVecB, false, SCL == 2>;
   constexpr int TA = StageA::kElems, TB = StageB::kElems, PB = StageB::kParts;
   __shared__ __align__(16) __bf16 smem[2 * (TA + TB)];
 
@@ -658,6 +688,8 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     ke = std::min<int64_t>(p.K, kb + p.k_per_split);
   }
 
+  // The wavefront's 64 or 32 rows share a sign (WM divides wm0).
+  const float unscale = A_KC && RowNegated(m0 + wm0) ? -kUnscale<PB> : kUnscale<PB>;
   floatx16 acc[BM][BN], sum[BM][BN];  // the current chunk's, and those before it
 #pragma unroll
   for (int i = 0; i < BM; ++i)
@@ -681,8 +713,8 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
       bf16x8 fa[BM][3], fb[BN][PB];
       ReadFrags<MT_N, KT, B_KC, BN, PB>(bs, wn0, g, lane, fb);
       ReadFrags<MT_M, KT, A_KC, BM, 3>(as, wm0, g, lane, fa);
-      if (decltype(fold)::value && g == 0) MfmaStep<true>(fa, fb, acc, sum);
-      else MfmaStep<false>(fa, fb, acc, sum);
+      if (decltype(fold)::value && g == 0) MfmaStep<true, A_KC>(fa, fb, acc, sum, unscale);
+      else MfmaStep<false, A_KC>(fa, fb, acc, sum, unscale);
     }
   };
   auto compute_at = [&](int64_t s) {  // stage s from its buffer
@@ -724,8 +756,12 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   // 8192x2048x2048: NT 128x64 428 | 402, 256x128 362 | 335; NN 128x128 of four
   // wavefronts 432 | 404, 256x128 362 | 348; TN 256x128 344 | 363; 128x64 NN
   // 530 | 545, TN 532 | 562).
-  constexpr int kSplitOps = BM * BN == 1 ? 28
-                            : VEC && (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
+  // The NT 128x128 tile of four wavefronts takes 30: at 40 it reloads a spilled
+  // register every chunk (2048x2048x2048 113 us at 40, 105 at 30).
+  constexpr int kSplitOps = BM * BN == 1                                   ? 28
+                            : !VEC                                         ? 24
+                            : kOneSet && A_KC && B_KC && NT == 256         ? 30
+                            : (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
                                                                            : 24;
   // Steady-state iteration on stage t (t + 2 < nfull): load stage t + 2 into
   // set `ld`, contract stage t, store stage t + 1 from set `st`. With VEC the
@@ -796,8 +832,8 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
         for (int i = 0; i < BM; ++i) {
           bf16x8 fa[1][3];
           ReadFrags<MT_M, KT, A_KC, 1, 3>(a_buf(cur), wm0 + 32 * i, 0, lane, fa);
-          MfmaStep<decltype(fold)::value>(fa, fb, reinterpret_cast<floatx16(&)[1][BN]>(acc[i]),
-                                          reinterpret_cast<floatx16(&)[1][BN]>(sum[i]));
+          MfmaStep<decltype(fold)::value, A_KC>(fa, fb, reinterpret_cast<floatx16(&)[1][BN]>(acc[i]),
+                                          reinterpret_cast<floatx16(&)[1][BN]>(sum[i]), unscale);
 #pragma unroll
           for (int v = kV * i / BM; v < kV * (i + 1) / BM; ++v) {
             if (v < kVA) {
@@ -879,7 +915,7 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
     for (int j = 0; j < BN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v)
-        acc[i][j][v] = __builtin_fmaf(acc[i][j][v], kUnscale<PB>, sum[i][j][v]);
+        acc[i][j][v] = __builtin_fmaf(acc[i][j][v], !A_KC && v & 1 ? -unscale : unscale, sum[i][j][v]);
 
   // Recompute: a non-finite block's outputs by fp32 products, straight from
   // memory (k pairs 16g + j, 16g + 8 + j). Decided per 32x32 block of the
@@ -932,13 +968,13 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
 #pragma unroll
       for (int j = 0; j < BN; ++j) {
         bf16x8 fa[1][3], fb[1][3];
-        Split8(tl[i], fa[0]);
-        Split8(tl[BM + j], fb[0]);
+        Split8(tl[i], fa[0], RowNegated(m0 + wm0) ? -kOpScale : kOpScale);
+        Split8(tl[BM + j], fb[0], kOpScale);
         floatx16 ua[1][1] = {}, before[1][1] = {};
-        MfmaStep<true>(fa, fb, ua, before);
+        MfmaStep<true, A_KC>(fa, fb, ua, before, unscale);
         floatx16& u = ua[0][0];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) u[v] *= kUnscale<3>;
+        for (int v = 0; v < 16; ++v) u[v] *= unscale;
         if (__builtin_expect(AnyNonFinite(u), false)) {
 #pragma unroll
           for (int v = 0; v < 16; ++v) u[v] = 0.0f;

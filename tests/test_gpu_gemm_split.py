@@ -235,3 +235,30 @@ def test_split_k_scratch_stays_within_the_covering_slices(gpu, wide):
                 assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (M, N, K)
                 served += 1
     assert served >= 6
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 16), (1024, 1024, 64), (1024, 256, 4096)])
+def test_errors_do_not_lean_to_one_side(gpu, M, N, K):
+    """The mean error stays within ten standard deviations of the mean of that
+    many independent errors, on every layout and tile config and in the LoRA
+    epilogue: a lean would add up in a sum over rows."""
+    torch, L = gpu
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    A, B = (torch.randn(*s, device="cuda:0", generator=g) for s in ((M, K), (K, N)))
+    want = A.double() @ B.double()
+
+    def check(out, what):
+        e = out.reshape(M, N).double() - want
+        assert float(e.mean().abs()) <= 10 * float(e.pow(2).mean().sqrt()) / (M * N) ** 0.5, what
+
+    out = torch.empty(M * N, device="cuda:0")
+    for layout in range(3):
+        a, b = A.T.contiguous() if layout == 2 else A, B.T.contiguous() if layout == 1 else B
+        for cfg in range(L.seeml_hip_gemm_config_count() - 1):
+            call(gpu, "gemm_forced", layout, a, b, out, M, N, K, cfg, 1)
+            check(out, (layout, cfg))
+    if K == 16:
+        zero, w = torch.zeros(M, 64, device="cuda:0"), torch.ones(N, 64, device="cuda:0")
+        for cfg in (0, 2, 4, 5, 8, 9):
+            call(gpu, "gemm_forced_lora", 1, zero, w, out, M, N, 64, cfg, 0, 0, A, B, K, 0, 1.0, 1)
+            check(out, cfg)
