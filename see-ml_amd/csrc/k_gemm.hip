@@ -151,6 +151,15 @@ int SplitsFor(const GemmDesc& d, SkinnyKind kind) {
   if (kind != SkinnyKind::kRowDot && kind != SkinnyKind::kColSum && mid > 64) most = mid < 256 ? d.K / 1024 : d.K / 2048;
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(CeilDiv(512, tiles), std::min<int64_t>(most, 64))));
 }
+
+// Whether the 16-byte form's 32-bit byte offsets reach the last row of a tile
+// of config `cfg`: k-contiguous rows of 2^22 elements and more are too far
+// apart for 256 of them (128, and row-contiguous ones, fit to 2^23).
+bool TileOffsetsFit(const GemmDesc& d, int cfg) {
+  constexpr int64_t kLong = int64_t{1} << 22;
+  return !(d.a_kc && d.lda >= kLong && kCfgs[cfg].mt_m > 128) &&
+         !(d.b_kc && d.ldb >= kLong && kCfgs[cfg].mt_n > 128);
+}
 }  // namespace
 
 GemmPlan PlanGemmWith(const GemmDesc& d, int forced_cfg, int forced_splits) {
@@ -172,6 +181,7 @@ GemmPlan PlanGemmWith(const GemmDesc& d, int forced_cfg, int forced_splits) {
   else
     plan.splits = SplitsFor(d, kind);
   plan.cfg = forced_cfg >= 0 && forced_cfg < kNumCfgs ? forced_cfg : TileFor(d, plan.splits);
+  if (!TileOffsetsFit(d, plan.cfg)) plan.cfg = gemm::kCfgDefault;
   plan.ws_bytes = plan.splits > 1 ? static_cast<size_t>(plan.splits) * d.M * d.N * sizeof(float) : 0;
   return plan;
 }
@@ -230,7 +240,7 @@ GemmPlan PlanGemmSplit(const GemmDesc& d, int cfg, int tail_cfg, int64_t n_split
       tail_cfg < 0 || tail_cfg >= kNumCfgs || plan.splits != 1 || !GemmVecForm(d))
     return plan;
   if (n_split <= 0) {
-    if (cfg != 2) return plan;
+    if (plan.cfg != gemm::kCfgLarge) return plan;
     const CfgInfo& c = kCfgs[cfg];
     const int64_t cus = DeviceCUs();
     const int64_t tm = CeilDiv(d.M, c.mt_m), bands = CeilDiv(d.N, c.mt_n);
@@ -249,7 +259,7 @@ GemmPlan PlanGemmSplit(const GemmDesc& d, int cfg, int tail_cfg, int64_t n_split
 bool GemmVecForm(const GemmDesc& d) {
   return !d.b_int8 && VecOk(d.A, d.lda, d.a_sb, d.a_sh, d.a_kc ? d.K : d.M) &&
          VecOk(d.B, d.ldb, d.b_sb, d.b_sh, d.b_kc ? d.K : d.N) &&
-         d.lda < (int64_t{1} << 22) && d.ldb < (int64_t{1} << 22);
+         d.lda < (int64_t{1} << 23) && d.ldb < (int64_t{1} << 23);
 }
 
 // Validates a tile-kernel launch of d under plan (one column range, no
@@ -290,6 +300,8 @@ Status PrepareKArgs(const GemmDesc& d, const GemmPlan& plan, const Ctx& ctx, Gem
   if (d.out && !vec && d.ldo && d.ldo != d.N)
     return Status::Fail(kUnitEngine, "Gemm: a column view's fused AddEW needs the 16-byte-load kernels");
   if (d.out && !vec) return Status::Fail(kUnitEngine, "Gemm: a fused AddEW needs the 16-byte-load kernels");
+  if (vec && !TileOffsetsFit(d, plan.cfg))
+    return Status::Fail(kUnitEngine, "Gemm: row strides too long for this tile config");
   const int cfg = vec ? plan.cfg : gemm::GeneralCfg(plan.cfg);
   const CfgInfo& c = kCfgs[cfg];
   const int64_t tm = CeilDiv(d.M, c.mt_m), tn = CeilDiv(d.N, c.mt_n);

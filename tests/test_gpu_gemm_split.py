@@ -262,3 +262,19 @@ def test_errors_do_not_lean_to_one_side(gpu, M, N, K):
         for cfg in (0, 2, 4, 5, 8, 9):
             call(gpu, "gemm_forced_lora", 1, zero, w, out, M, N, 64, cfg, 0, 0, A, B, K, 0, 1.0, 1)
             check(out, cfg)
+
+
+def test_rows_four_million_elements_apart_keep_the_vector_form(gpu):
+    """k-contiguous rows of 2^22 to 2^23 elements: 32-bit byte offsets reach 128
+    of them, so a 256-row tile gives way to the 128-row one, in the 16-byte form
+    that the LoRA epilogue needs."""
+    torch, _ = gpu
+    M, N, K, rank = 300, 64, (1 << 22) + 4, 16
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    A, B, T, Bl = (torch.randn(*s, device="cuda:0", generator=g) for s in ((M, K), (N, K), (M, rank), (rank, N)))
+    out = torch.empty(M, N, device="cuda:0")
+    call(gpu, "gemm_forced_lora", 1, A, B, out, M, N, K, 2, 0, 0, T, Bl, rank, 0, 1.0, 1)
+    want = T.double() @ Bl.double()
+    for k in range(0, K, 1 << 18):
+        want += A[:, k:k + (1 << 18)].double() @ B[:, k:k + (1 << 18)].double().T
+    assert float((out.double() - want).norm()) <= bound(K) * float(want.norm())
