@@ -175,11 +175,11 @@ SKINNY = [
 
 
 def heuristic_splits(M, N, K):
-    """The untuned plan's split-K count for a batch-1 GEMM (PlanGemmWith,
-    csrc/k_gemm.hip): its tile (128x32 for N <= 32, 32x128 for M <= 32,
-    else 128x128 or, when that leaves few tiles or an extent <= 64, 64x64);
-    fewer than 512 tiles and K >= 256 split K so the slices cover the chip
-    twice, each at least 128 deep."""
+    """Split-K slices that cover the chip twice, each at least 128 deep: by
+    128x128 tiles, or 64x64 ones where those are many or an extent is <= 64
+    (128x32 for N <= 32, 32x128 for M <= 32); one below K = 256 or from 512
+    tiles on. The untuned plan's count for the rank-wide shapes, and a bound
+    on it for every other (SplitsFor, csrc/k_gemm.hip)."""
     cdiv = lambda a, b: -(-a // b)
     if N <= 32 < M:
         mt = (128, 32)
