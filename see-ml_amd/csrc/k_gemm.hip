@@ -409,7 +409,7 @@ Status LaunchGemm(const GemmDesc& d, const GemmPlan& plan, const Ctx& ctx) {
   if (Status s = CheckEpilogue(d, plan); !s) return s;
   const bool vec_form = GemmVecForm(d);
   if (d.out && !d.lora_t && !vec_form && !d.out_scaled && !(d.ldo && d.ldo != d.N)) {
-    // The element-load form has no fused epilogue: the GEMM stores C (always
+    // The general form has no fused epilogue: the GEMM stores C (always
     // safe: C's range is C's while the GEMM writes it), then the AddEW runs.
     GemmDesc plain = d;
     plain.addend = nullptr;

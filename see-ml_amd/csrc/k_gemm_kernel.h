@@ -37,15 +37,15 @@
 // accumulator is added to a second one and cleared every 64 k (kChunk), which
 // keeps the rounding small. The bf16 MFMA's own additions lean to one side;
 // half of the rows are computed negated, so that a sum over many rows of such
-// results does not add the lean up (RowNegated below). Relative 2-norm error against 64 bits, fp32 MFMA | this: normal
-// operands K = 16 7.4e-8 | 3.3e-8, K = 2048 8.1e-7 | 1.6e-7, K = 8192 1.62e-6 |
-// 2.5e-7; softmax gradients times a head of 8192 classes 1.6e-6 | 2.3e-7;
-// log-normal operands 6.6e-7 | 1.3e-7 (without the second accumulator 7.0e-7
-// on the second, and gradients summed over 2048 rows were further off than
-// with the fp32 MFMA). An int8 operand is one bf16 part: three products.
+// results does not add the lean up (RowNegated below). Relative 2-norm error
+// against 64 bits, fp32 MFMA | this: normal operands K = 16 7.4e-8 | 3.3e-8,
+// K = 2048 8.1e-7 | 1.6e-7, K = 8192 1.62e-6 | 2.5e-7 (without the second
+// accumulator 7.0e-7 at K = 2048); softmax gradients times a head of 8192
+// classes 1.6e-6 | 2.3e-7; log-normal operands 6.6e-7 | 1.3e-7. An int8 operand
+// is one bf16 part: three products.
 // Measured: NT 8192x2048x5504 1330 -> 854 us, 8192x5504x2048 1334 -> 921 us,
 // 200-216 TFLOP/s of fp32 products where 157 was the fp32 MFMA's peak. What
-// bounds it now is power: the matrix cores are 76% busy at 1.74 GHz (2.4 with
+// bounds it now is power: the matrix cores are 70% busy at 1.78 GHz (2.4 with
 // little to do), and a loop of bf16 MFMAs alone on random bits runs at the
 // clock that makes 300.
 //
@@ -1050,12 +1050,7 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   // activation or causal zeroing): one base pointer per lane, every element
   // a compile-time number of rows and columns from it, no per-element bounds
   // or epilogue branches. Stores what the general write-back below stores.
-  // The 128x128x32/w2x2 tile keeps the general write-back: two of its
-  // workgroups share a CU, the other's k loop hides this one's write-back,
-  // and the back-to-back stores measured ~1% slower on it in the C4 step.
-  constexpr bool kPlainFast =
-      VEC && !(MT_M == 128 && MT_N == 128 && KT == 32 && WAVES_M == 2 && WAVES_N == 2);
-  if constexpr (kPlainFast) {
+  if constexpr (VEC) {
     if (!p.out && p.splits == 1 && !p.accumulate && !p.bias && p.act == 0 &&
         p.causal != static_cast<int>(Causal::kLowerOut) && m0 + MT_M <= p.M &&
         n0 + MT_N <= p.N) {

@@ -1,4 +1,4 @@
-// k_gemm_q8.hip — GEMM kernel instantiations: int8 B (GemmNNQ8 / GemmNTQ8), element loads.
+// k_gemm_q8.hip — GEMM kernel instantiations: int8 B (GemmNNQ8 / GemmNTQ8), the general load form.
 #include "k_gemm_kernel.h"
 
 namespace seeml_hip {

@@ -50,7 +50,7 @@ def main(argv=None):
     libs = [(x.split("=", 1)[0], bind(x.split("=", 1)[1])) for x in a.libs] or [("tree", bind(_lib.LIB_PATH))]
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(3)
-    cfg = 2  # 256x128x32/w4x2
+    cfg = 2  # 256x128x16/w4x2
     cases = []
     for lay, M, N, K in SHAPES:
         ops = dict(A=torch.randn(M, K, device=dev, generator=g),
@@ -97,7 +97,7 @@ def main(argv=None):
                     ts.append(e0.elapsed_time(e1) / reps * 1e3)
                 res.setdefault((ln, nm, kind), []).append(statistics.median(ts))
         print(f"epilogue_ab: round {rnd + 1}/{a.rounds}", flush=True)
-    print(f"epilogue_ab: {'cold' if a.cold else 'warm'} operands, tile 256x128x32/w4x2, median us per launch")
+    print(f"epilogue_ab: {'cold' if a.cold else 'warm'} operands, tile 256x128x16/w4x2, median us per launch")
     head = "".join(f" {ln:>10s} {'vs plain':>9s}" for ln, _ in libs)
     print(f"{'shape':22s} {'epilogue':8s}{head}")
     for nm, kind, _ in cases:
