@@ -756,10 +756,12 @@ __device__ __forceinline__ void gemm_tile(const GemmKArgs& p, uint32_t L, uint32
   // 8192x2048x2048: NT 128x64 428 | 402, 256x128 362 | 335; NN 128x128 of four
   // wavefronts 432 | 404, 256x128 362 | 348; TN 256x128 344 | 363; 128x64 NN
   // 530 | 545, TN 532 | 562).
+  // With int8 B it is 20 (2048x2048x2048 NN and NT 77.6 and 66.9 us at 24, 79.3
+  // and 63.5 at 20; 8192x2048x2048 284 and 257, 282 and 243).
   // The NT 128x128 tile of four wavefronts takes 30: at 40 it reloads a spilled
   // register every chunk (2048x2048x2048 113 us at 40, 105 at 30).
   constexpr int kSplitOps = BM * BN == 1                                   ? 28
-                            : !VEC                                         ? 24
+                            : !VEC                                         ? (PB == 1 ? 20 : 24)
                             : kOneSet && A_KC && B_KC && NT == 256         ? 30
                             : (kOneSet ? A_KC || NT == 256 : A_KC && B_KC) ? 40
                                                                            : 24;
